@@ -31,7 +31,7 @@ namespace tempi {
 namespace {
 
 struct BatchItem {
-  int32_t kind;            // 4 * variant + 2 * aligned + direction
+  int32_t kind;            // 4 * variant + 2 * whole rows + direction
   uint32_t units_per_tile; // units of one block-pass: groups per block * K
   uint32_t ntiles;         // tiles of this request
   uint32_t pad;
@@ -47,11 +47,11 @@ constexpr uint32_t kXcds = 8;
 // neighbouring blocks measured about 0.2 us faster per launch on MI355X for
 // 12-B rows 2 KiB apart (262 144 rows), the same as the single-copy kernels'
 // grid-stride order.
-template <int P, int W, int U, bool ALIGNED, int DIR, bool NTS, bool NTL>
+template <int P, int W, int U, bool WHOLE, int DIR, bool NTS, bool NTL>
 __device__ __forceinline__ void copy_tile(const KParams &p, uint32_t l,
                                           uint32_t nt) {
   constexpr uint32_t GROUPS = kBlock / P;
-  copy_units<P, W, U, ALIGNED, DIR, NTS, NTL>(p, l * GROUPS + threadIdx.x / P,
+  copy_units<P, W, U, WHOLE, DIR, NTS, NTL>(p, l * GROUPS + threadIdx.x / P,
                                               nt * GROUPS, p.units,
                                               threadIdx.x % P);
 }
@@ -247,12 +247,12 @@ int plan_batch(const std::vector<Req> &rs, int cu_count, BatchPlan *pl) {
   uint64_t tiles = 0;
   for (const Req &r : rs) {
     BatchItem it{};
-    bool aligned = false;
-    int err = fill_kparams(r.g, r.ds, r.dp, r.dir, r.variant, &it.p, &aligned);
+    bool whole = false;
+    int err = fill_kparams(r.g, r.ds, r.dp, r.dir, r.variant, &it.p, &whole);
     if (err) {
       return err;
     }
-    it.kind = 4 * r.variant + 2 * (aligned ? 1 : 0) + r.dir;
+    it.kind = 4 * r.variant + 2 * (whole ? 1 : 0) + r.dir;
     const VariantDesc &v = kVariants[r.variant];
     it.units_per_tile = (uint32_t)(kBlock / v.P) * units_in_flight(v.U);
     const uint64_t t = ((uint64_t)it.p.units + it.units_per_tile - 1) /

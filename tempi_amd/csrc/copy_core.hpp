@@ -4,9 +4,11 @@
 // A copy is `units` work units; unit u is segment (u % nseg) of row
 // (u / nseg).  A group of P lanes moves one unit as U words of W bytes per
 // lane, the P lanes touching consecutive words; each thread issues the loads
-// of K = units_in_flight(U) units before storing any of them.  Stores are always aligned
-// to the word's natural unit A (W for powers of two, 4 for 12-byte words);
-// loads may sit at any byte address (gfx9 global loads accept that).
+// of K = units_in_flight(U) units before storing any of them.  Loads and
+// stores may sit at any byte address (gfx9 global memory instructions accept
+// that), so a row's words are counted from its first byte whatever its
+// alignment, and the L % W bytes after the last whole word are the same for
+// every row of a copy: one lane moves them as 8, 4, 2 and 1 bytes.
 #pragma once
 
 #include "internal.hpp"
@@ -43,6 +45,7 @@ struct KParams {
   FastDiv div[kMaxRowDims];
   int64_t str[kMaxRowDims];
   uint32_t signal; // nonzero: the launch signals its completion (kernels.hip)
+  uint32_t tail;   // L % W
 };
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -57,11 +60,6 @@ template <> struct WordT<4> { typedef uint32_t T; };
 template <> struct WordT<2> { typedef uint16_t T; };
 template <> struct WordT<1> { typedef uint8_t T; };
 
-// alignment unit of a W-byte word
-__host__ __device__ constexpr int word_align(int W) {
-  return (W & (W - 1)) == 0 ? W : 4;
-}
-
 // load W bytes from any byte address; NT marks the load nontemporal (the
 // line is filled for this access and is first in line for eviction)
 template <int W, bool NT>
@@ -75,47 +73,15 @@ __device__ __forceinline__ typename WordT<W>::T load_word(const char *p) {
   }
 }
 
-// store W bytes to an address aligned to word_align(W)
+// store W bytes to any byte address
 template <int W, bool NT>
 __device__ __forceinline__ void store_word(char *p, typename WordT<W>::T v) {
   typedef typename WordT<W>::T T;
-  typedef T Ta __attribute__((aligned(word_align(W))));
+  typedef T Tu __attribute__((aligned(1)));
   if constexpr (NT) {
-    __builtin_nontemporal_store(v, reinterpret_cast<Ta *>(p));
+    __builtin_nontemporal_store(v, reinterpret_cast<Tu *>(p));
   } else {
-    *reinterpret_cast<Ta *>(p) = v;
-  }
-}
-
-// Copy n < 16 bytes to d from s (any alignment) with the widest stores d's
-// alignment allows: 1, 2, 4 then 8 bytes on the way up to an aligned
-// address, 8, 4, 2 then 1 on the way down from one (at most four stores
-// either way).
-__device__ __forceinline__ void copy_short(char *d, const char *s,
-                                           uint32_t n) {
-  while (n) {
-    const uintptr_t a = (uintptr_t)d;
-    if ((a & 1) || n < 2) {
-      *d = *s;
-      d += 1;
-      s += 1;
-      n -= 1;
-    } else if ((a & 2) || n < 4) {
-      store_word<2, false>(d, load_word<2, false>(s));
-      d += 2;
-      s += 2;
-      n -= 2;
-    } else if ((a & 4) || n < 8) {
-      store_word<4, false>(d, load_word<4, false>(s));
-      d += 4;
-      s += 4;
-      n -= 4;
-    } else {
-      store_word<8, false>(d, load_word<8, false>(s));
-      d += 8;
-      s += 8;
-      n -= 8;
-    }
+    *reinterpret_cast<Tu *>(p) = v;
   }
 }
 
@@ -140,36 +106,23 @@ __host__ __device__ __forceinline__ int64_t row_offset(const KParams &p,
   return off;
 }
 
-// How unit_addr moves the head and tail bytes of a misaligned row: the
-// kernels copy them (DeviceMem); the host-side emulation of a copy records
-// the bytes instead (kernels.hip), so one definition of the address
-// arithmetic serves both.
-struct DeviceMem {
-  __device__ static __forceinline__ void copy_short(char *d, const char *s,
-                                                    uint32_t n) {
-    ::tempi::copy_short(d, s, n);
-  }
-  __device__ static __forceinline__ void copy_byte(char *d, const char *s) {
-    *d = *s;
-  }
-};
-
 // Addresses of one work unit, computed before any of the thread's loads.
 struct UnitAddr {
-  const char *s; // first body byte on the source side
-  char *d;       // first body byte on the destination side
+  const char *s; // first byte of the row on the source side
+  char *d;       // first byte of the row on the destination side
   uint32_t w;    // first word index of this lane
-  uint32_t n;    // body words of the row (0: nothing to move)
+  uint32_t n;    // words of the row (0: nothing to move)
+  bool tail;     // this lane moves the row's last L % W bytes
 };
 
 // Address phase of work unit `u` (wave-uniform when P == 64).  DIR 0 = pack
-// (strided -> packed), 1 = unpack (packed -> strided).  Head and tail bytes
-// of a row whose destination is not word-aligned are copied here directly.
-template <class M, int P, int W, int U, bool ALIGNED, int DIR>
+// (strided -> packed), 1 = unpack (packed -> strided).  A row's last segment
+// holds its tail; the lane that would move the next word moves it.  The
+// host-side emulation of a copy (kernels.hip) runs the same code.
+template <int P, int W, int U, bool WHOLE, int DIR>
 __host__ __device__ __forceinline__ UnitAddr unit_addr(const KParams &p,
                                                        uint32_t u,
                                                        uint32_t lane) {
-  constexpr int A = word_align(W);
   const uint32_t row = p.nseg == 1 ? u : p.segdiv.div(u);
   const uint32_t seg = u - row * p.nseg;
   const int64_t soff = row_offset(p, row);
@@ -178,35 +131,72 @@ __host__ __device__ __forceinline__ UnitAddr unit_addr(const KParams &p,
   a.s = p.src + (DIR == 0 ? soff : poff);
   a.d = p.dst + (DIR == 0 ? poff : soff);
   a.w = seg * (uint32_t)(P * U) + lane;
-  if constexpr (ALIGNED) {
-    a.n = p.words;
-  } else {
-    const uint32_t mis = (uint32_t)((uintptr_t)a.d & (A - 1));
-    uint32_t head = mis ? (uint32_t)(A - mis) : 0u;
-    if ((int64_t)head > p.L) {
-      head = (uint32_t)p.L;
-    }
-    a.n = (uint32_t)((p.L - head) / W);
-    if (seg == 0) {
-      const int64_t t0 = (int64_t)head + (int64_t)a.n * W;
-      const uint32_t tail = (uint32_t)(p.L - t0);
-      if constexpr (P == 1) {
-        // one lane per row: the widest aligned stores, at most four each
-        M::copy_short(a.d, a.s, head);
-        M::copy_short(a.d + t0, a.s + t0, tail);
-      } else {
-        for (uint32_t b = lane; b < head; b += P) {
-          M::copy_byte(a.d + b, a.s + b);
-        }
-        for (uint32_t b = lane; b < tail; b += P) {
-          M::copy_byte(a.d + t0 + b, a.s + t0 + b);
-        }
-      }
-    }
-    a.s += head;
-    a.d += head;
-  }
+  a.n = p.words;
+  a.tail = !WHOLE && seg == p.nseg - 1 && lane == p.words % P;
   return a;
+}
+
+// Byte offset, within a row's tail of `tail` bytes, of its piece of N bytes
+// (N = 8, 4, 2 or 1, present when the bit N of `tail` is set): after the
+// larger pieces.
+template <int N>
+__host__ __device__ constexpr uint32_t tail_at(uint32_t tail) {
+  return tail & ~(uint32_t)(2 * N - 1);
+}
+
+// The tails of K units in registers, between the load and the store phase.
+// `tail` is the same for every row, so the tests of its bits do not diverge.
+template <int W> struct TailWords {
+  u32x2 v8;
+  uint32_t v4;
+  uint16_t v2;
+  uint8_t v1;
+};
+
+template <int W, bool NT>
+__device__ __forceinline__ void load_tail(TailWords<W> *t, const char *s,
+                                          uint32_t tail) {
+  if constexpr (W > 8) {
+    if (tail & 8) {
+      t->v8 = load_word<8, NT>(s);
+    }
+  }
+  if constexpr (W > 4) {
+    if (tail & 4) {
+      t->v4 = load_word<4, NT>(s + tail_at<4>(tail));
+    }
+  }
+  if constexpr (W > 2) {
+    if (tail & 2) {
+      t->v2 = load_word<2, NT>(s + tail_at<2>(tail));
+    }
+  }
+  if (tail & 1) {
+    t->v1 = load_word<1, NT>(s + tail_at<1>(tail));
+  }
+}
+
+template <int W, bool NT>
+__device__ __forceinline__ void store_tail(const TailWords<W> &t, char *d,
+                                           uint32_t tail) {
+  if constexpr (W > 8) {
+    if (tail & 8) {
+      store_word<8, NT>(d, t.v8);
+    }
+  }
+  if constexpr (W > 4) {
+    if (tail & 4) {
+      store_word<4, NT>(d + tail_at<4>(tail), t.v4);
+    }
+  }
+  if constexpr (W > 2) {
+    if (tail & 2) {
+      store_word<2, NT>(d + tail_at<2>(tail), t.v2);
+    }
+  }
+  if (tail & 1) {
+    store_word<1, NT>(d + tail_at<1>(tail), t.v1);
+  }
 }
 
 // s_waitcnt immediate for vmcnt(0) alone on gfx9 (expcnt and lgkmcnt at
@@ -230,7 +220,7 @@ __host__ __device__ constexpr int units_in_flight(int U) {
 // in front of the later ones (register reuse across the grid-stride loop),
 // and each unit paid a full memory round trip of its own.  NTS / NTL:
 // nontemporal stores / loads of the body words.
-template <int P, int W, int U, bool ALIGNED, int DIR, bool NTS, bool NTL>
+template <int P, int W, int U, bool WHOLE, int DIR, bool NTS, bool NTL>
 __device__ __forceinline__ void copy_units(const KParams &p, uint32_t first,
                                            uint32_t stride, uint32_t end,
                                            uint32_t lane) {
@@ -245,12 +235,13 @@ __device__ __forceinline__ void copy_units(const KParams &p, uint32_t first,
       u = __builtin_amdgcn_readfirstlane(u);
     }
     if (u < end) {
-      a[k] = unit_addr<DeviceMem, P, W, U, ALIGNED, DIR>(p, u, lane);
+      a[k] = unit_addr<P, W, U, WHOLE, DIR>(p, u, lane);
     } else {
       a[k].s = nullptr;
       a[k].d = nullptr;
       a[k].w = 0;
       a[k].n = 0;
+      a[k].tail = false;
     }
   }
   UnitWords<W, U> v[K];
@@ -261,6 +252,16 @@ __device__ __forceinline__ void copy_units(const KParams &p, uint32_t first,
       const uint32_t w = a[k].w + j * P;
       if (w < a[k].n) {
         v[k].v[j] = load_word<W, NTL>(a[k].s + (size_t)w * W);
+      }
+    }
+  }
+  TailWords<W> t[K];
+  const int64_t tail_off = (int64_t)p.words * W;
+  if constexpr (!WHOLE) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      if (a[k].tail) {
+        load_tail<W, NTL>(&t[k], a[k].s + tail_off, p.tail);
       }
     }
   }
@@ -277,6 +278,14 @@ __device__ __forceinline__ void copy_units(const KParams &p, uint32_t first,
       const uint32_t w = a[k].w + j * P;
       if (w < a[k].n) {
         store_word<W, NTS>(a[k].d + (size_t)w * W, v[k].v[j]);
+      }
+    }
+  }
+  if constexpr (!WHOLE) {
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      if (a[k].tail) {
+        store_tail<W, NTS>(t[k], a[k].d + tail_off, p.tail);
       }
     }
   }
@@ -313,9 +322,10 @@ constexpr int kBlock = 256;
 // copy along its outer row dimensions.
 constexpr int64_t kMaxUnits = 1ll << 31;
 
-// Fill the kernel parameters of one copy with `variant`; a copy of
-// kMaxUnits units or more is reported as TEMPI_ERR_UNSUPPORTED.
+// Fill the kernel parameters of one copy with `variant`; `whole`: its rows
+// are whole words.  A copy of kMaxUnits units or more is reported as
+// TEMPI_ERR_UNSUPPORTED.
 int fill_kparams(const Geom &g, const char *strided, char *packed, int dir,
-                 int variant, KParams *p, bool *aligned);
+                 int variant, KParams *p, bool *whole);
 
 } // namespace tempi

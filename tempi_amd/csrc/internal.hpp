@@ -225,9 +225,9 @@ struct VariantDesc {
 extern const VariantDesc kVariants[];
 extern const int kNumVariants;
 
-// true when every row starts W-aligned on both sides and L % W == 0
+// true when every row starts at a multiple of A on both sides and L % A == 0
 bool geom_aligned(const Geom &g, const char *strided, const char *packed,
-                  int W);
+                  int A);
 
 // enqueue the copy; `strided` / `packed` are device addresses of the
 // buffer origin (strided) and of the first packed byte.

@@ -5,12 +5,20 @@
 // internal.hpp).  A work unit is one segment of one row; a group of P lanes
 // of a 64-wide wavefront moves a segment as U words of W bytes per lane, the
 // P lanes of a group touching consecutive words so that each load and store
-// instruction of the group covers P*W contiguous bytes.  The stores are
-// always W-aligned: when the store side of a row does not start W-aligned,
-// the lanes copy the head and tail bytes one at a time and the body words are
-// loaded from wherever they sit on the other side (gfx9 global loads accept
-// any byte alignment).  When the host has shown that both sides of every row
-// are W-aligned and L % W == 0, the ALIGNED instantiation skips that logic.
+// instruction of the group covers P*W contiguous bytes.  gfx950's global
+// loads and stores accept any byte address, so neither side's alignment
+// changes how a row is cut: its words start at its first byte and its last
+// L % W bytes are a tail of at most four pieces, the same for every row.  An
+// earlier form stored only to W-aligned addresses and copied the head and
+// tail bytes of each row one by one, every byte its own store and most of
+// them a round trip of their own.  Unpacks by the same variant, three buffer
+// pairs in turn, the strided side 5 B past a boundary, before and now:
+//   2^20 rows of 32 B at a 512-B stride    67.5 -> 28.4 us  (variant 5)
+//   2^19 rows of 64 B at a 1777-B stride   44.9 -> 34.4 us  (variant 5)
+//   2^17 rows of 256 B at a 700-B stride   27.4 -> 22.5 us  (variant 10)
+//   2^16 rows of 512 B at a 3000-B stride  24.7 -> 19.4 us  (variant 10)
+// What is left is the traffic of partial lines.
+// When L % W == 0 the WHOLE instantiation has no tail.
 //
 // reference: include/pack_kernels.cuh:19-120 (grid_x_memcpy_aligned,
 // pack_2d/unpack_2d) and :350-433 (pack_3d/unpack_3d).  The index map is the
@@ -84,7 +92,7 @@ __device__ __forceinline__ void signal_done(const KParams &p) {
   }
 }
 
-template <int P, int W, int U, bool ALIGNED, int DIR, bool NTS, bool NTL>
+template <int P, int W, int U, bool WHOLE, int DIR, bool NTS, bool NTL>
 __global__ void __launch_bounds__(kBlock) k_strided_copy(KParams p) {
   constexpr uint32_t GROUPS = kBlock / P;
   constexpr uint32_t K = units_in_flight(U);
@@ -92,7 +100,7 @@ __global__ void __launch_bounds__(kBlock) k_strided_copy(KParams p) {
   const uint32_t step = gridDim.x * GROUPS;
   for (uint32_t u = blockIdx.x * GROUPS + threadIdx.x / P; u < p.units;
        u += step * K) {
-    copy_units<P, W, U, ALIGNED, DIR, NTS, NTL>(p, u, step, p.units, lane);
+    copy_units<P, W, U, WHOLE, DIR, NTS, NTL>(p, u, step, p.units, lane);
   }
   signal_done(p);
 }
@@ -114,7 +122,7 @@ typedef void (*KernelFn)(KParams);
    {k_strided_copy<P, W, U, true, 0, NTS, NTL>,                                \
     k_strided_copy<P, W, U, true, 1, NTS, NTL>}},
 
-// [variant][aligned][dir]
+// [variant][whole rows][dir]
 static const KernelFn kKernels[][2][2] = {TEMPI_VARIANTS(TEMPI_KROW)};
 #undef TEMPI_KROW
 static_assert(sizeof(kKernels) / sizeof(kKernels[0]) ==
@@ -177,9 +185,8 @@ int make_geom(const tempi_strided_block &sb, int64_t count, Geom *g) {
 }
 
 bool geom_aligned(const Geom &g, const char *strided, const char *packed,
-                  int W) {
-  const int A = word_align(W);
-  if (g.L % W) {
+                  int A) {
+  if (g.L % A) {
     return false;
   }
   if ((uintptr_t)packed % A || (uintptr_t)(strided + g.start) % A) {
@@ -245,9 +252,9 @@ int heuristic_variant(const Geom &g, const char *strided, const char *packed,
 }
 
 int fill_kparams(const Geom &g, const char *strided, char *packed, int dir,
-                 int variant, KParams *pp, bool *aligned) {
+                 int variant, KParams *pp, bool *whole) {
   const VariantDesc &v = kVariants[variant];
-  *aligned = geom_aligned(g, strided, packed, v.W);
+  *whole = g.L % v.W == 0;
   const int64_t words = g.L / v.W;
   const int64_t per_unit = (int64_t)v.P * v.U;
   const int64_t nseg = std::max<int64_t>(1, (words + per_unit - 1) / per_unit);
@@ -272,6 +279,7 @@ int fill_kparams(const Geom &g, const char *strided, char *packed, int dir,
   p.nseg = (uint32_t)nseg;
   p.segdiv = make_fastdiv((uint32_t)nseg);
   p.words = (uint32_t)words;
+  p.tail = (uint32_t)(g.L % v.W);
   p.nrd = g.nrd;
   for (int k = 0; k < g.nrd; ++k) {
     if (g.cnt[k] >= (1ll << 32)) {
@@ -378,13 +386,13 @@ static int launch_one(const Geom &g, const char *strided, char *packed,
                       int dir, int variant, hipStream_t stream,
                       int max_blocks, bool signal = false) {
   KParams p;
-  bool aligned = false;
-  int err = fill_kparams(g, strided, packed, dir, variant, &p, &aligned);
+  bool whole = false;
+  int err = fill_kparams(g, strided, packed, dir, variant, &p, &whole);
   if (err) {
     return err;
   }
   const int64_t blocks = grid_of(variant, p.units, max_blocks, device_cu_count());
-  KernelFn fn = kKernels[variant][aligned ? 1 : 0][dir];
+  KernelFn fn = kKernels[variant][whole ? 1 : 0][dir];
   p.signal = signal ? 1u : 0u;
   void *args[] = {&p};
   TEMPI_HIP_CHECK(hipLaunchKernel(reinterpret_cast<const void *>(fn),
@@ -693,29 +701,31 @@ struct Recorder {
 
 thread_local Recorder *t_rec = nullptr;
 
-struct HostMem {
-  static void copy_short(char *d, const char *s, uint32_t n) {
-    t_rec->read(s, n);
-    t_rec->write(d, n);
-  }
-  static void copy_byte(char *d, const char *s) {
-    t_rec->read(s, 1);
-    t_rec->write(d, 1);
-  }
-};
-
 // one work unit of one group, all P lanes: the kernels' address phase, then
-// the body words of the load and store phases
-template <int P, int W, int U, bool ALIGNED, int DIR>
+// the words and tail pieces of the load and store phases
+template <int P, int W, int U, bool WHOLE, int DIR>
 void emulate_unit(const KParams &p, uint32_t u) {
   for (uint32_t lane = 0; lane < (uint32_t)P; ++lane) {
-    const UnitAddr a = unit_addr<HostMem, P, W, U, ALIGNED, DIR>(p, u, lane);
+    const UnitAddr a = unit_addr<P, W, U, WHOLE, DIR>(p, u, lane);
     for (int j = 0; j < U; ++j) {
       const uint32_t w = a.w + (uint32_t)(j * P);
       if (w < a.n) {
         t_rec->read(a.s + (size_t)w * W, W);
         t_rec->write(a.d + (size_t)w * W, W);
       }
+    }
+    if (!WHOLE && a.tail) {
+      const int64_t off = (int64_t)p.words * W;
+      const auto piece = [&](uint32_t n, uint32_t at) {
+        if (p.tail & n) {
+          t_rec->read(a.s + off + at, n);
+          t_rec->write(a.d + off + at, n);
+        }
+      };
+      piece(8, 0);
+      piece(4, tail_at<4>(p.tail));
+      piece(2, tail_at<2>(p.tail));
+      piece(1, tail_at<1>(p.tail));
     }
   }
 }
@@ -815,13 +825,13 @@ TEMPI_EXPORT int tempi_copy_emulate(const tempi_strided_block *sb,
       g, strided, packed, variant,
       [&](const Geom &pg, const char *ps, char *pp) -> int {
         KParams p;
-        bool aligned = false;
-        int e = fill_kparams(pg, ps, pp, direction, variant, &p, &aligned);
+        bool whole = false;
+        int e = fill_kparams(pg, ps, pp, direction, variant, &p, &whole);
         if (e) {
           return e;
         }
         const VariantDesc &v = kVariants[variant];
-        const EmulateFn fn = kEmulate[variant][aligned ? 1 : 0][direction];
+        const EmulateFn fn = kEmulate[variant][whole ? 1 : 0][direction];
         const uint32_t GROUPS = (uint32_t)(kBlock / v.P);
         const uint32_t K = (uint32_t)units_in_flight(v.U);
         const uint32_t blocks =
