@@ -233,19 +233,26 @@ bool geom_aligned(const Geom &g, const char *strided, const char *packed,
 // buffer origin (strided) and of the first packed byte.
 int launch_copy(const Geom &g, const char *strided, char *packed, int dir,
                 int variant, hipStream_t stream, int max_blocks = 0);
-// launch_copy on the library stream, then wait until the copy is done (a
-// copy of a few workgroups signals its own completion to the host)
+// launch_copy on the library stream, then wait until the copy is done
 int launch_copy_wait(const Geom &g, const char *strided, char *packed, int dir,
                      int variant, int max_blocks = 0);
-// launch_copy on the library stream without waiting; a copy that signals
-// its completion gets *seq > 0, to test with signal_reached (else 0)
+// launch_copy on the library stream without waiting; *seq > 0: the number of
+// the signal to test for with signal_reached (0: wait on the stream); *own:
+// the copy's last workgroup sends it
 int launch_copy_signalled(const Geom &g, const char *strided, char *packed,
                           int dir, int variant, int max_blocks,
-                          unsigned long long *seq);
+                          unsigned long long *seq, bool *own);
+// the number of a signal sent once everything on the library stream so far
+// is done; 0: there is none
+unsigned long long signal_stream();
 bool signal_reached(unsigned long long seq);
-// until signal `seq` arrives (seq 0: none) or `ev`, recorded after the
-// copy, completes; a failed event is an error
-int wait_signal_or_event(unsigned long long seq, hipEvent_t ev);
+// has signal `seq` arrived (0: is the library stream done)?  `polls` counts
+// the caller's calls
+int poll_signal_or_stream(unsigned long long seq, uint32_t *polls, bool *done);
+// until signal `seq` arrives (0: until the library stream is done)
+int wait_signal_or_stream(unsigned long long seq);
+// until everything on the library stream is done
+int wait_library_stream();
 
 // closed-form variant rule (the "plain heuristic")
 int heuristic_variant(const Geom &g, const char *strided, const char *packed,
@@ -413,10 +420,10 @@ int run_copy(const tempi_strided_block &sb, int64_t count, const char *strided,
 // the copy is done (launch_copy_wait)
 int run_copy_wait(const tempi_strided_block &sb, int64_t count,
                   const char *strided, char *packed, int dir);
-// the same without waiting; *seq > 0 when the copy signals its completion
+// the same without waiting; *seq and *own as for launch_copy_signalled
 int run_copy_signalled(const tempi_strided_block &sb, int64_t count,
                        const char *strided, char *packed, int dir,
-                       unsigned long long *seq);
+                       unsigned long long *seq, bool *own);
 
 // cached staging buffers (pool.cpp): device memory, or pinned host memory
 // mapped into the device address space

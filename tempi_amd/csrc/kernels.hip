@@ -54,9 +54,8 @@ FastDiv make_fastdiv(uint32_t d) {
 // host; set once by the host (signal_ready) before the first signalled
 // launch.
 struct SignalSlots {
-  unsigned long long *counter;   // finished workgroups of the running launch
-  unsigned long long *completed; // signalled launches completed so far
-  unsigned long long *flag;      // `completed`, in pinned host memory
+  uint32_t *counter; // finished workgroups of the running launch
+  uint32_t *flag;    // number of the last completed signal, in pinned host memory
 };
 static __device__ SignalSlots g_signal_slots;
 
@@ -65,31 +64,35 @@ static __device__ SignalSlots g_signal_slots;
 // barrier's workgroup-scope fences order the other waves' stores before
 // thread 0's release, scopes composing), then counted.  The launch's last
 // workgroup resets the counter for the next signalled launch -- launches on
-// the library stream never overlap -- and stores the number of completed
-// signalled launches to the host's flag.
+// the library stream never overlap -- and stores the launch's number to the
+// host's flag.  The count itself is relaxed: the fences before and after it
+// order it, and an ordered one would write the L2 back a second time per
+// workgroup (128 workgroups of 16 KiB, launch to flag: 11.5 -> 10.7 us).
 __device__ __forceinline__ void signal_done(const KParams &p) {
   if (!p.signal) {
     return;
   }
+  const SignalSlots s = g_signal_slots;
   __syncthreads();
   if (threadIdx.x == 0) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
-    const SignalSlots s = g_signal_slots;
-    const unsigned long long done =
-        __hip_atomic_fetch_add(s.counter, 1ull, __ATOMIC_ACQ_REL,
-                               __HIP_MEMORY_SCOPE_AGENT) +
-        1ull;
+    const uint32_t done = __hip_atomic_fetch_add(s.counter, 1u, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT) +
+                          1u;
     if (done == gridDim.x) {
-      __hip_atomic_store(s.counter, 0ull, __ATOMIC_RELAXED,
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "");
+      __hip_atomic_store(s.counter, 0u, __ATOMIC_RELAXED,
                          __HIP_MEMORY_SCOPE_AGENT);
-      const unsigned long long c =
-          __hip_atomic_fetch_add(s.completed, 1ull, __ATOMIC_RELAXED,
-                                 __HIP_MEMORY_SCOPE_AGENT) +
-          1ull;
-      __hip_atomic_store(s.flag, c, __ATOMIC_RELEASE,
+      __hip_atomic_store(s.flag, p.signal, __ATOMIC_RELEASE,
                          __HIP_MEMORY_SCOPE_SYSTEM);
     }
   }
+}
+
+// A signal of its own: launched after the work it reports on the same
+// stream, which has finished, its stores written back, when this starts.
+__global__ void k_signal(uint32_t *flag, uint32_t number) {
+  __hip_atomic_store(flag, number, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 template <int P, int W, int U, bool WHOLE, int DIR, bool NTS, bool NTL>
@@ -380,11 +383,11 @@ static int for_each_launch(const Geom &g, const char *strided, char *packed,
   return TEMPI_SUCCESS;
 }
 
-// One launch; `signal`: it signals its completion (the caller holds the
-// signal's lock).
+// One launch; `signal` > 0: it signals its completion with that number (the
+// caller holds the signal's lock).
 static int launch_one(const Geom &g, const char *strided, char *packed,
                       int dir, int variant, hipStream_t stream,
-                      int max_blocks, bool signal = false) {
+                      int max_blocks, uint32_t signal = 0) {
   KParams p;
   bool whole = false;
   int err = fill_kparams(g, strided, packed, dir, variant, &p, &whole);
@@ -393,7 +396,7 @@ static int launch_one(const Geom &g, const char *strided, char *packed,
   }
   const int64_t blocks = grid_of(variant, p.units, max_blocks, device_cu_count());
   KernelFn fn = kKernels[variant][whole ? 1 : 0][dir];
-  p.signal = signal ? 1u : 0u;
+  p.signal = signal;
   void *args[] = {&p};
   TEMPI_HIP_CHECK(hipLaunchKernel(reinterpret_cast<const void *>(fn),
                                   dim3((unsigned)blocks), dim3(kBlock), args,
@@ -440,22 +443,28 @@ int launch_copy(const Geom &g, const char *strided, char *packed, int dir,
 // but hipStreamSynchronize returns after 11.1 us: the rest is the runtime's
 // end-of-kernel processing.  A copy of one launch of at most
 // kSignalMaxBlocks workgroups on the library stream therefore signals its
-// own completion (KParams::signal) and the host spins on the flag.  Larger
-// grids wait on the stream: the workgroups' releases and counter updates
-// queue behind each other, and past about 150 of them they cost more than
-// the wait saves (MPI_Pack of 64-B rows: 12.5-13.1 us signalled against
-// 13.3-13.7 us at 128 workgroups, 14.9 against 13.7 us at 192).
+// own completion (KParams::signal) and the host spins on the flag.  In larger
+// grids each workgroup's release writes its XCD's L2 back and those queue
+// behind each other (counting in 32 leaves instead of one counter changes
+// nothing), so a one-thread kernel behind the copy stores the flag instead: it
+// starts after the copy's own end-of-kernel write-back.  Copies of 16 KiB per
+// workgroup, launch to the host seeing it, us:
+//   workgroups               64    128    256    512   1024   2048
+//   own signal              8.9   10.7   14.3   21.9   37.2   72.1
+//   signal kernel behind    9.9   10.0   10.2   10.8   11.2   17.2
+//   hipStreamSynchronize   11.9   12.2   12.5   13.4   14.5   20.8
 
 namespace {
 
 constexpr int64_t kSignalMaxBlocks = 128;
 
 struct SignalState {
-  std::mutex mu; // held from a launch's sequence number to its launch
+  std::mutex mu; // held from a signal's number to its launch
   bool tried = false;
-  unsigned long long *slots = nullptr;    // device memory: counter, completed
-  unsigned long long *flag = nullptr;     // pinned host memory
-  unsigned long long issued = 0;          // signalled launches so far
+  uint32_t *counter = nullptr;  // device memory
+  uint32_t *flag = nullptr;     // pinned host memory
+  uint32_t *flag_dev = nullptr; // its device address
+  unsigned long long issued = 0; // signals so far
   // set after a signalled wait fails: the counter may no longer match the
   // launches, so later copies wait on the stream
   std::atomic<bool> off{false};
@@ -466,15 +475,27 @@ SignalState &signal_state() {
   return s;
 }
 
-// Counter, completed count and flag, allocated and published to the kernels
-// once, on the library stream's device (the state's lock held); false when
-// they cannot be.
+// The kernels store the low 32 bits of a signal's number; the next number
+// skips those that would read as none (the state's lock held).
+unsigned long long next_signal(const SignalState &st) {
+  const unsigned long long n = st.issued + 1;
+  return (uint32_t)n ? n : n + 1;
+}
+
+bool flag_at(const SignalState &st, unsigned long long seq) {
+  // fewer than 2^31 signals are ever in flight
+  return (int32_t)(__atomic_load_n(st.flag, __ATOMIC_ACQUIRE) -
+                   (uint32_t)seq) >= 0;
+}
+
+// Counter and flag, allocated and published to the kernels once, on the
+// library stream's device (the state's lock held); false when they cannot be.
 bool signal_ready(SignalState &st) {
   if (st.tried) {
     return st.flag != nullptr && !st.off.load(std::memory_order_relaxed);
   }
   st.tried = true;
-  // the zeroed counters and the published slots are in place before the
+  // the zeroed counter and the published slots are in place before the
   // first signalled launch: both go through the library stream (which does
   // not wait for the null stream), and it is drained here
   hipStream_t s = library_stream();
@@ -485,9 +506,9 @@ bool signal_ready(SignalState &st) {
                                                      hipHostMallocPortable) &&
             hipSuccess == hipHostGetDevicePointer(&fd, f, 0);
   if (ok) {
-    __atomic_store_n(static_cast<unsigned long long *>(f), 0ull, __ATOMIC_RELEASE);
-    unsigned long long *cs = static_cast<unsigned long long *>(c);
-    const SignalSlots slots{cs, cs + 1, static_cast<unsigned long long *>(fd)};
+    __atomic_store_n(static_cast<uint32_t *>(f), 0u, __ATOMIC_RELEASE);
+    const SignalSlots slots{static_cast<uint32_t *>(c),
+                            static_cast<uint32_t *>(fd)};
     ok = hipSuccess == hipMemcpyToSymbolAsync(HIP_SYMBOL(g_signal_slots), &slots,
                                               sizeof slots, 0,
                                               hipMemcpyHostToDevice, s) &&
@@ -504,21 +525,22 @@ bool signal_ready(SignalState &st) {
     TEMPI_LOG(LOG_WARN, "no completion signal: synchronous copies wait on the stream");
     return false;
   }
-  st.slots = static_cast<unsigned long long *>(c);
-  st.flag = static_cast<unsigned long long *>(f);
+  st.counter = static_cast<uint32_t *>(c);
+  st.flag_dev = static_cast<uint32_t *>(fd);
+  st.flag = static_cast<uint32_t *>(f);
   return true;
 }
 
-// Spin until the flag counts `seq` completed signalled launches.  A launch
-// that never runs to its end leaves the flag short, so after 0.2 ms the
-// stream is checked every 0.1 ms: finished without the flag is an error,
-// and so is a failed stream.
-int wait_signal(const SignalState &st, unsigned long long seq,
-                hipStream_t stream) {
+// Spin until signal `seq` arrived.  A launch that never runs to its end
+// leaves the flag short, so after 0.2 ms the stream is checked every 0.1 ms:
+// finished without the flag is an error, and so is a failed stream.  An
+// error switches the signal off.
+int wait_signal(SignalState &st, unsigned long long seq) {
   const auto t0 = std::chrono::steady_clock::now();
   double check_at = 2e-4;
+  int err = TEMPI_SUCCESS;
   for (;;) {
-    if (__atomic_load_n(st.flag, __ATOMIC_ACQUIRE) >= seq) {
+    if (flag_at(st, seq)) {
       return TEMPI_SUCCESS;
     }
     __builtin_ia32_pause();
@@ -528,38 +550,67 @@ int wait_signal(const SignalState &st, unsigned long long seq,
     if (el < check_at) {
       continue;
     }
-    const hipError_t e = hipStreamQuery(stream);
+    const hipError_t e = hipStreamQuery(library_stream());
     if (e == hipSuccess) {
-      if (__atomic_load_n(st.flag, __ATOMIC_ACQUIRE) >= seq) {
+      if (flag_at(st, seq)) {
         return TEMPI_SUCCESS;
       }
-      return set_error(TEMPI_ERR_HIP, "a copy ended without its signal");
+      err = set_error(TEMPI_ERR_HIP, "a copy ended without its signal");
+      break;
     }
     if (e != hipErrorNotReady) {
       (void)hipGetLastError();
-      return set_error(TEMPI_ERR_HIP, "copy failed: %s", hipGetErrorString(e));
+      err = set_error(TEMPI_ERR_HIP, "copy failed: %s", hipGetErrorString(e));
+      break;
     }
     check_at = el + 1e-4;
   }
+  st.off.store(true);
+  TEMPI_LOG(LOG_WARN, "completion signal switched off: %s", tempi_last_error());
+  (void)hipStreamSynchronize(library_stream());
+  return err;
+}
+
+bool on_library_device() {
+  int dev = -1;
+  return hipSuccess == hipGetDevice(&dev) && dev == library_device();
 }
 
 // one launch of at most kSignalMaxBlocks workgroups, on the library
 // stream's device
 bool signal_fits(const Geom &g, int variant, int max_blocks) {
   const int64_t units = g.rows * segments_of(g, variant);
-  int dev = -1;
   return g.L <= (1ll << 30) && units < kMaxUnits &&
          grid_of(variant, (uint32_t)units, max_blocks, device_cu_count()) <=
              kSignalMaxBlocks &&
-         hipSuccess == hipGetDevice(&dev) && dev == library_device();
+         on_library_device();
 }
 
 } // namespace
 
+unsigned long long signal_stream() {
+  if (!on_library_device()) {
+    return 0;
+  }
+  SignalState &st = signal_state();
+  std::lock_guard<std::mutex> lk(st.mu);
+  if (!signal_ready(st)) {
+    return 0;
+  }
+  const unsigned long long n = next_signal(st);
+  hipLaunchKernelGGL(k_signal, dim3(1), dim3(1), 0, library_stream(),
+                     st.flag_dev, (uint32_t)n);
+  if (hipSuccess != hipGetLastError()) {
+    return 0;
+  }
+  return st.issued = n;
+}
+
 int launch_copy_signalled(const Geom &g, const char *strided, char *packed,
                           int dir, int variant, int max_blocks,
-                          unsigned long long *seq) {
+                          unsigned long long *seq, bool *own) {
   *seq = 0;
+  *own = false;
   if (g.rows == 0 || g.L == 0) {
     return TEMPI_SUCCESS;
   }
@@ -571,87 +622,79 @@ int launch_copy_signalled(const Geom &g, const char *strided, char *packed,
     SignalState &st = signal_state();
     std::lock_guard<std::mutex> lk(st.mu);
     if (signal_ready(st)) {
+      const unsigned long long n = next_signal(st);
       const int err = launch_one(g, strided, packed, dir, variant, s,
-                                 max_blocks, /*signal=*/true);
+                                 max_blocks, (uint32_t)n);
       if (!err) {
-        *seq = ++st.issued;
+        *seq = st.issued = n;
+        *own = true;
       }
       return err;
     }
   }
-  return launch_copy(g, strided, packed, dir, variant, s, max_blocks);
+  const int err = launch_copy(g, strided, packed, dir, variant, s, max_blocks);
+  if (!err) {
+    *seq = signal_stream();
+  }
+  return err;
 }
 
 bool signal_reached(unsigned long long seq) {
   const SignalState &st = signal_state();
-  return seq && st.flag && __atomic_load_n(st.flag, __ATOMIC_ACQUIRE) >= seq;
+  return seq && st.flag && flag_at(st, seq);
 }
 
-int wait_signal_or_event(unsigned long long seq, hipEvent_t ev) {
-  const auto t0 = std::chrono::steady_clock::now();
-  double check_at = seq ? 2e-4 : 0.0;
-  for (;;) {
-    if (signal_reached(seq)) {
-      ++counters().signalled_waits;
-      return TEMPI_SUCCESS;
-    }
-    __builtin_ia32_pause();
-    const double el = std::chrono::duration<double>(
-                          std::chrono::steady_clock::now() - t0)
-                          .count();
-    if (el < check_at) {
-      continue;
-    }
-    const hipError_t q = seq ? hipEventQuery(ev) : hipEventSynchronize(ev);
-    if (q == hipSuccess) {
-      return TEMPI_SUCCESS;
-    }
-    if (q != hipErrorNotReady) {
-      (void)hipGetLastError();
-      return set_error(TEMPI_ERR_HIP, "copy failed: %s", hipGetErrorString(q));
-    }
-    check_at = el + 1e-4;
+int poll_signal_or_stream(unsigned long long seq, uint32_t *polls, bool *done) {
+  *done = signal_reached(seq);
+  // a signal that does not come is looked after in the stream's own state,
+  // every so many polls: the query costs as much as hundreds of them
+  if (*done || (seq && ++*polls % 1024)) {
+    return TEMPI_SUCCESS;
   }
+  const hipError_t q = hipStreamQuery(library_stream());
+  if (q == hipErrorNotReady) {
+    return TEMPI_SUCCESS;
+  }
+  if (q != hipSuccess) {
+    (void)hipGetLastError();
+    return set_error(TEMPI_ERR_HIP, "copy failed: %s", hipGetErrorString(q));
+  }
+  *done = !seq || signal_reached(seq);
+  return *done ? TEMPI_SUCCESS
+               : set_error(TEMPI_ERR_HIP, "a copy ended without its signal");
 }
+
+int wait_signal_or_stream(unsigned long long seq) {
+  if (seq) {
+    return wait_signal(signal_state(), seq);
+  }
+  TEMPI_HIP_CHECK(hipStreamSynchronize(library_stream()));
+  return TEMPI_SUCCESS;
+}
+
+int wait_library_stream() { return wait_signal_or_stream(signal_stream()); }
 
 int launch_copy_wait(const Geom &g, const char *strided, char *packed,
                      int dir, int variant, int max_blocks) {
+  unsigned long long seq = 0;
+  bool own = false;
+  int err = launch_copy_signalled(g, strided, packed, dir, variant, max_blocks,
+                                  &seq, &own);
+  if (err) {
+    // part of the copy may be running
+    (void)hipStreamSynchronize(library_stream());
+    return err;
+  }
   if (g.rows == 0 || g.L == 0) {
     return TEMPI_SUCCESS;
   }
-  if (variant < 0 || variant >= kNumVariants) {
-    return set_error(TEMPI_ERR_ARG, "variant %d out of range", variant);
+  if ((err = wait_signal_or_stream(seq))) {
+    return err;
   }
-  hipStream_t s = library_stream();
-  if (signal_fits(g, variant, max_blocks)) {
-    SignalState &st = signal_state();
-    std::unique_lock<std::mutex> lk(st.mu);
-    if (signal_ready(st)) {
-      int err = launch_one(g, strided, packed, dir, variant, s, max_blocks,
-                           /*signal=*/true);
-      const unsigned long long seq = err ? st.issued : ++st.issued;
-      lk.unlock();
-      if (!err) {
-        err = wait_signal(st, seq, s);
-        if (err) {
-          st.off.store(true);
-          TEMPI_LOG(LOG_WARN, "completion signal switched off: %s",
-                    tempi_last_error());
-        }
-      }
-      if (err) {
-        (void)hipStreamSynchronize(s);
-        return err;
-      }
-      ++counters().signalled_waits;
-      return TEMPI_SUCCESS;
-    }
+  if (own) {
+    ++counters().signalled_waits;
   }
-  int err = launch_copy(g, strided, packed, dir, variant, s, max_blocks);
-  if (hipSuccess != hipStreamSynchronize(s) && !err) {
-    err = set_error(TEMPI_ERR_HIP, "stream synchronize failed");
-  }
-  return err;
+  return TEMPI_SUCCESS;
 }
 
 // ---------------------------------------------------------------------------

@@ -203,8 +203,8 @@ int run(Exchange &e, MPI_Comm comm) {
                                    s)) {
     err = set_error(TEMPI_ERR_HIP, "staging copy failed");
   }
-  if (!err && hipSuccess != hipStreamSynchronize(s)) {
-    err = set_error(TEMPI_ERR_HIP, "pack for MPI_Neighbor_alltoallw failed");
+  if (!err) {
+    err = wait_library_stream();
   }
   if (err) {
     return MPI_ERR_INTERN;
@@ -226,8 +226,8 @@ int run(Exchange &e, MPI_Comm comm) {
     return MPI_ERR_INTERN;
   }
   err = tempi_batch_launch(e.unpack, s);
-  if (!err && hipSuccess != hipStreamSynchronize(s)) {
-    err = set_error(TEMPI_ERR_HIP, "unpack for MPI_Neighbor_alltoallw failed");
+  if (!err) {
+    err = wait_library_stream();
   }
   return err ? MPI_ERR_INTERN : MPI_SUCCESS;
 }

@@ -353,8 +353,9 @@ bool library_cannot_read(const void *buf, int count, int peer) {
 class IsendOp : public AsyncOp {
   enum { PACKING, SENDING, DONE } state_ = PACKING;
   Staging stg_;
-  hipEvent_t ev_ = nullptr;
   unsigned long long seq_ = 0; // the pack's completion signal (0: none)
+  bool own_ = false;           // the pack's own workgroups send it
+  uint32_t polls_ = 0;
   MPI_Request lib_req_ = MPI_REQUEST_NULL;
   int64_t bytes_;
   int peer_, tag_;
@@ -374,9 +375,6 @@ public:
       // never completed (an error path): the pack may still be running
       (void)hipStreamSynchronize(library_stream());
     }
-    if (ev_) {
-      (void)hipEventDestroy(ev_);
-    }
     stg_.release();
   }
   bool is_send() const override { return true; }
@@ -384,17 +382,11 @@ public:
     hipStream_t s = library_stream();
     int err = stg_.acquire(method, bytes_);
     if (!err && method != TEMPI_METHOD_STAGED) {
-      // the pack is all there is to wait for: it may signal its completion
       err = run_copy_signalled(cn.sb, count, static_cast<const char *>(ubuf_dev),
-                               stg_.kernel_side(), TEMPI_DIR_PACK, &seq_);
+                               stg_.kernel_side(), TEMPI_DIR_PACK, &seq_, &own_);
     } else if (!err) {
       err = enqueue_pack(cn, count, ubuf_dev, stg_, s);
-    }
-    if (!err && hipSuccess != hipEventCreateWithFlags(&ev_, hipEventDisableTiming)) {
-      err = set_error(TEMPI_ERR_HIP, "event creation failed");
-    }
-    if (!err && hipSuccess != hipEventRecord(ev_, s)) {
-      err = set_error(TEMPI_ERR_HIP, "event record failed");
+      seq_ = err ? 0 : signal_stream();
     }
     return err;
   }
@@ -402,29 +394,26 @@ public:
     if (state_ != PACKING) {
       return MPI_SUCCESS;
     }
-    if (signal_reached(seq_)) {
-      ++counters().signalled_waits;
-      return post();
-    }
-    const hipError_t q = hipEventQuery(ev_);
-    if (q == hipErrorNotReady) {
-      return MPI_SUCCESS;
-    }
-    if (q != hipSuccess) {
-      set_error(TEMPI_ERR_HIP, "pack for MPI_Isend failed: %s",
-                hipGetErrorString(q));
+    bool done = false;
+    if (poll_signal_or_stream(seq_, &polls_, &done)) {
+      TEMPI_LOG(LOG_ERROR, "pack for MPI_Isend: %s", tempi_last_error());
       return MPI_ERR_INTERN;
     }
+    if (!done) {
+      return MPI_SUCCESS;
+    }
+    counters().signalled_waits += own_;
     return post();
   }
   int post_blocking() override {
     if (state_ != PACKING) {
       return MPI_SUCCESS;
     }
-    if (wait_signal_or_event(seq_, ev_)) {
+    if (wait_signal_or_stream(seq_)) {
       TEMPI_LOG(LOG_ERROR, "pack for MPI_Isend: %s", tempi_last_error());
       return MPI_ERR_INTERN;
     }
+    counters().signalled_waits += own_;
     return post();
   }
   bool done() const override { return state_ == DONE; }
@@ -454,8 +443,9 @@ public:
 class IrecvOp : public AsyncOp {
   enum { RECEIVING, UNPACKING, DONE } state_ = RECEIVING;
   Staging stg_;
-  hipEvent_t ev_ = nullptr;
   unsigned long long seq_ = 0; // the unpack's completion signal (0: none)
+  bool own_ = false;           // the unpack's own workgroups send it
+  uint32_t polls_ = 0;
   MPI_Request lib_req_ = MPI_REQUEST_NULL;
   MPI_Status status_{};
   Canon cn_;
@@ -474,12 +464,11 @@ class IrecvOp : public AsyncOp {
     int err = TEMPI_SUCCESS;
     if (stg_.method != TEMPI_METHOD_STAGED) {
       err = run_copy_signalled(cn_.sb, n, static_cast<const char *>(ubuf_dev_),
-                               stg_.kernel_side(), TEMPI_DIR_UNPACK, &seq_);
+                               stg_.kernel_side(), TEMPI_DIR_UNPACK, &seq_,
+                               &own_);
     } else {
       err = enqueue_unpack(cn_, n, ubuf_dev_, stg_, (int64_t)n * cn_.size, s);
-    }
-    if (!err && hipSuccess != hipEventRecord(ev_, s)) {
-      err = set_error(TEMPI_ERR_HIP, "event record failed");
+      seq_ = err ? 0 : signal_stream();
     }
     return mpi_error_of(err);
   }
@@ -491,18 +480,11 @@ public:
     if (state_ == UNPACKING) {
       (void)hipStreamSynchronize(library_stream());
     }
-    if (ev_) {
-      (void)hipEventDestroy(ev_);
-    }
     stg_.release();
   }
   bool is_send() const override { return false; }
   int start(int method, int peer, int tag, MPI_Comm comm) {
-    int err = stg_.acquire(method, bytes_);
-    if (!err && hipSuccess != hipEventCreateWithFlags(&ev_, hipEventDisableTiming)) {
-      err = set_error(TEMPI_ERR_HIP, "event creation failed");
-    }
-    if (err) {
+    if (stg_.acquire(method, bytes_)) {
       return MPI_ERR_INTERN;
     }
     return real_mpi().Irecv(stg_.wire(), (int)bytes_, MPI_PACKED, peer, tag,
@@ -525,17 +507,14 @@ public:
         state_ = DONE;
         return error_;
       }
-      if (signal_reached(seq_)) {
-        ++counters().signalled_waits;
-        state_ = DONE;
-        return MPI_SUCCESS;
-      }
-      const hipError_t q = hipEventQuery(ev_);
-      if (q == hipSuccess) {
-        state_ = DONE;
-      } else if (q != hipErrorNotReady) {
-        set_error(TEMPI_ERR_HIP, "unpack for MPI_Irecv failed");
+      bool done = false;
+      if (poll_signal_or_stream(seq_, &polls_, &done)) {
+        TEMPI_LOG(LOG_ERROR, "unpack for MPI_Irecv: %s", tempi_last_error());
         return MPI_ERR_INTERN;
+      }
+      if (done) {
+        counters().signalled_waits += own_;
+        state_ = DONE;
       }
     }
     return MPI_SUCCESS;
@@ -563,10 +542,13 @@ public:
         error_ = uerr;
       }
     }
-    if (state_ == UNPACKING && error_ == MPI_SUCCESS &&
-        wait_signal_or_event(seq_, ev_)) {
-      TEMPI_LOG(LOG_ERROR, "unpack for MPI_Irecv: %s", tempi_last_error());
-      error_ = MPI_ERR_INTERN;
+    if (state_ == UNPACKING && error_ == MPI_SUCCESS) {
+      if (wait_signal_or_stream(seq_)) {
+        TEMPI_LOG(LOG_ERROR, "unpack for MPI_Irecv: %s", tempi_last_error());
+        error_ = MPI_ERR_INTERN;
+      } else {
+        counters().signalled_waits += own_;
+      }
     }
     state_ = DONE;
     if (st != MPI_STATUS_IGNORE) {
@@ -835,8 +817,8 @@ TEMPI_EXPORT int MPI_Send(const void *buf, int count, MPI_Datatype datatype,
                          st.kernel_side(), TEMPI_DIR_PACK);
   } else if (!terr) {
     terr = enqueue_pack(cn, count, dev, st, s);
-    if (!terr && hipSuccess != hipStreamSynchronize(s)) {
-      terr = set_error(TEMPI_ERR_HIP, "pack for MPI_Send failed");
+    if (!terr) {
+      terr = wait_library_stream();
     }
   }
   if (terr) {
@@ -909,8 +891,8 @@ TEMPI_EXPORT int MPI_Recv(void *buf, int count, MPI_Datatype datatype,
                            st.kernel_side(), TEMPI_DIR_UNPACK);
     } else {
       terr = enqueue_unpack(cn, n, dev, st, (int64_t)n * cn.size, s);
-      if (!terr && hipSuccess != hipStreamSynchronize(s)) {
-        terr = set_error(TEMPI_ERR_HIP, "unpack for MPI_Recv failed");
+      if (!terr) {
+        terr = wait_library_stream();
       }
     }
     if (terr) {
