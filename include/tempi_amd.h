@@ -172,11 +172,12 @@ int tempi_variant_info_get(int variant, tempi_variant_info *info);
 #define TEMPI_SELECT_DEFAULT 3   /* library policy (model if loaded)    */
 
 /* Variant the library would use for this copy.  Under the default policy a
-   copy of 64 MiB or more is settled on its first run: the model's three
-   best variants and the closed-form rule's pick are each timed once, cold,
-   writing a scratch image of the destination (never the caller's buffers),
-   and the fastest is kept for the shape; before that run this returns the
-   model's pick. */
+   copy of at most 1 MiB (128 KiB in rows under 64 B) takes a closed-form
+   choice: it is bound by its launch, not by the kernel.  A copy of 64 MiB or
+   more is settled on its first run: the model's three best variants and the
+   closed-form rule's pick are each timed once, cold, writing a scratch image
+   of the destination (never the caller's buffers), and the fastest is kept
+   for the shape; before that run this returns the model's pick. */
 int tempi_select_variant(const tempi_strided_block *sb, int64_t incount,
                          const void *strided_buf, const void *packed_buf,
                          int direction, int method, int *variant);

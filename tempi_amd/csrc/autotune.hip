@@ -353,8 +353,13 @@ static int verify_candidates(const Geom &g, const char *strided, char *packed,
 }
 
 Choice choose(const Geom &g, const char *strided, char *packed, int dir,
-              int method, hipStream_t stream, bool in_place) {
+              int method, hipStream_t stream, CopyUse use) {
+  const bool in_place = use == CopyUse::kNext;
   Choice c;
+  if (method == TEMPI_SELECT_DEFAULT && use != CopyUse::kInBatch &&
+      (c.variant = latency_variant(g)) >= 0) {
+    return c;
+  }
   c.variant = heuristic_variant(g, strided, packed, dir);
   if (method == TEMPI_SELECT_MODEL ||
       (method == TEMPI_SELECT_DEFAULT && model_available())) {

@@ -520,7 +520,7 @@ TEMPI_EXPORT int tempi_batch_create(const tempi_batch_request *reqs, int64_t n,
   for (Req &q : rs) {
     if (q.variant < 0) {
       q.variant = choose(q.g, q.ds, q.dp, q.dir, method, library_stream(),
-                         /*in_place=*/false)
+                         CopyUse::kInBatch)
                       .variant;
     }
   }

@@ -258,19 +258,28 @@ int wait_library_stream();
 int heuristic_variant(const Geom &g, const char *strided, const char *packed,
                       int dir);
 
+// the variant for a copy that runs alone and is bound by its launch; -1: it
+// is too large for that
+int latency_variant(const Geom &g);
+
 // a kernel variant and its grid cap (0: the default cap)
 struct Choice {
   int variant = 0;
   int max_blocks = 0;
 };
 
+// What a chosen variant is for: the copy that runs next on the caller's
+// buffers, one request of a batch that is being created, or an answer to a
+// query.
+enum class CopyUse { kNext, kInBatch, kQuery };
+
 // variant selection entry used by the MPI and tempi_* paths; AUTOTUNE (and
 // the default policy for copies of 64 MiB or more) times candidates on
-// `stream` (results cached by shape): on the caller's buffers when
-// `in_place` (the copy itself runs next, writing the same bytes), else on a
-// scratch image of the written side
+// `stream` (results cached by shape): on the caller's buffers when the copy
+// runs next (it writes the same bytes), else on a scratch image of the
+// written side
 Choice choose(const Geom &g, const char *strided, char *packed, int dir,
-              int method, hipStream_t stream, bool in_place);
+              int method, hipStream_t stream, CopyUse use);
 
 // grid caps the autotuner tries, as multiples of the CU count (0 = default)
 extern const int kGridCaps[];

@@ -192,7 +192,7 @@ int run_copy(const tempi_strided_block &sb, int64_t count, const char *strided,
   Choice c;
   if (variant < 0) {
     c = choose(g, strided, packed, dir, env().select, stream,
-               /*in_place=*/true);
+               CopyUse::kNext);
   } else {
     c.variant = variant;
   }
@@ -211,7 +211,7 @@ int run_copy_wait(const tempi_strided_block &sb, int64_t count,
     return TEMPI_SUCCESS;
   }
   const Choice c = choose(g, strided, packed, dir, env().select,
-                          library_stream(), /*in_place=*/true);
+                          library_stream(), CopyUse::kNext);
   return launch_copy_wait(g, strided, packed, dir, c.variant, c.max_blocks);
 }
 
@@ -231,7 +231,7 @@ int run_copy_signalled(const tempi_strided_block &sb, int64_t count,
     return TEMPI_SUCCESS;
   }
   const Choice c = choose(g, strided, packed, dir, env().select,
-                          library_stream(), /*in_place=*/true);
+                          library_stream(), CopyUse::kNext);
   return launch_copy_signalled(g, strided, packed, dir, c.variant,
                                c.max_blocks, seq, own);
 }
@@ -651,13 +651,13 @@ TEMPI_EXPORT int tempi_select_variant(const tempi_strided_block *sb,
       return set_error(TEMPI_ERR_ARG, "autotuning needs device-accessible buffers");
     }
     *variant = choose(g, static_cast<const char *>(ds), static_cast<char *>(dp),
-                      direction, method, library_stream(), /*in_place=*/false)
+                      direction, method, library_stream(), CopyUse::kQuery)
                    .variant;
     return TEMPI_SUCCESS;
   }
   *variant = choose(g, static_cast<const char *>(strided_buf),
                     static_cast<char *>(const_cast<void *>(packed_buf)),
-                    direction, method, nullptr, /*in_place=*/false)
+                    direction, method, nullptr, CopyUse::kQuery)
                  .variant;
   return TEMPI_SUCCESS;
 }

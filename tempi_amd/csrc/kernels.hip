@@ -254,6 +254,44 @@ int heuristic_variant(const Geom &g, const char *strided, const char *packed,
   return L >= 16 ? 7 : 11;
 }
 
+// Launched back to back, all variants move a copy of up to 1 MiB at the
+// launch cadence (2.2-2.6 us on MI355X), which leaves the selector nothing to
+// rank; waited for, the one with the fewest workgroups and the widest words
+// that cut no row is seen first.  MPI_Pack, us (workgroups):
+//   1024 rows of 256 B   variant 4 9.5 (32), 10 9.7 (64), 1 10.7 (256)
+//   8192 rows of 64 B    variant 6 10.0 (64), 4 10.4 (256), 9 11.8 (128)
+//   1024 rows of 1 KiB   variant 4 10.1 (64), 1 10.3 (256), 7 11.3 (64)
+//   4096 rows of 24 B    variant 8 10.4 (32), 10 11.3 (512), 1 12.6 (2048)
+//   300 rows of 12 B     variants 9, 12 9.0 (2, 1), 7 9.8 (2), 1 10.6 (75)
+// Rows under 64 B leave this regime earlier: the kernel's own time shows
+// (64 Ki rows of 12 B: variants 9 11.3, 12 11.9, 4 12.7, 1 21.9 us), so beyond
+// 128 KiB they stay with the selector.
+int latency_variant(const Geom &g) {
+  const int64_t L = g.L, bytes = g.L * g.rows;
+  if (bytes > (L < 64 ? 128ll << 10 : 1ll << 20)) {
+    return -1;
+  }
+  if (L >= 256) {
+    return 4;
+  }
+  if (L >= 128) {
+    return 5;
+  }
+  if (L >= 64 || L == 48) {
+    return 6;
+  }
+  if (L % 16 == 0) {
+    return 7;
+  }
+  if (L % 8 == 0) {
+    return 8;
+  }
+  if (L % 12 == 0) {
+    return 12;
+  }
+  return L % 4 == 0 || L < 16 ? 9 : 7;
+}
+
 int fill_kparams(const Geom &g, const char *strided, char *packed, int dir,
                  int variant, KParams *pp, bool *whole) {
   const VariantDesc &v = kVariants[variant];

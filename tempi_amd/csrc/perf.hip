@@ -797,7 +797,7 @@ int measure_table(int table, const Sampling &sampling, Table *out) {
       const char *sp = static_cast<const char *>(strided.p);
       char *pp = static_cast<char *>(packed_dev);
       const Choice ch = choose(g, sp, pp, dir, env().select, s,
-                               /*in_place=*/true);
+                               CopyUse::kNext);
       IidTime r;
       err = sample_point(
           [&](double *tm) -> int {
