@@ -157,8 +157,9 @@ typedef struct tempi_variant_info {
   int32_t lanes_per_row; /* lanes of a wavefront that share one row   */
   int32_t word_bytes;    /* bytes per load/store                      */
   int32_t unroll;        /* words each lane moves per work unit       */
-  int32_t nontemporal_stores; /* stores marked nontemporal           */
-  int32_t nontemporal_loads;  /* loads marked nontemporal            */
+  int32_t nontemporal_stores; /* an unpack's stores marked nontemporal */
+  int32_t nontemporal_loads;  /* loads marked nontemporal (a pack's only,
+                                 when nontemporal_stores is set too)   */
 } tempi_variant_info;
 int tempi_num_variants(void);
 int tempi_variant_info_get(int variant, tempi_variant_info *info);

@@ -313,13 +313,22 @@ int trial_buffers(const Geom &g, const char *strided, char *packed, int dir,
 static int verify_candidates(const Geom &g, const char *strided, char *packed,
                              int dir, int rule, hipStream_t stream,
                              bool in_place, Choice *out) {
-  int cand[4];
-  int n = model_ranked(g, strided, packed, dir, 3, cand);
-  if (n == 0) {
+  int ranked[3];
+  const int m = model_ranked(g, strided, packed, dir, 3, ranked);
+  if (m == 0) {
     return TEMPI_ERR_UNSUPPORTED;
   }
-  if (std::find(cand, cand + n, rule) == cand + n) {
-    cand[n++] = rule;
+  int cand[4];
+  int n = 0;
+  cand[n++] = rule;
+  for (int i = 0; i < m; ++i) {
+    // which accesses are nontemporal shows in the kernels that run next, not
+    // in a copy timed alone: the rule decides it, the trials the rest
+    const int v =
+        streamed_variant(ranked[i], g, strided, dir, touched_bytes(g));
+    if (std::find(cand, cand + n, v) == cand + n) {
+      cand[n++] = v;
+    }
   }
   TrialBuffers t;
   const char *ts = strided;
@@ -382,7 +391,13 @@ Choice choose(const Geom &g, const char *strided, char *packed, int dir,
     }
     const int v = model_variant(g, strided, packed, dir, key);
     if (v >= 0) {
-      c.variant = v;
+      // requests of a batch share lines with each other (a halo's faces,
+      // edges and corners): nontemporal loads would read those again
+      c.variant =
+          method == TEMPI_SELECT_DEFAULT
+              ? streamed_variant(v, g, strided, dir,
+                                 use == CopyUse::kInBatch ? 0 : touched_bytes(g))
+              : v;
     }
     return c;
   }

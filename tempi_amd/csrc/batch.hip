@@ -59,21 +59,22 @@ __device__ __forceinline__ void copy_tile(const KParams &p, uint32_t l,
 __device__ __forceinline__ void run_tile(int kind, const KParams &p,
                                          uint32_t l, uint32_t nt) {
   switch (kind) {
-#define TEMPI_BCASE(I, P, W, U, NTS, NTL)                                      \
+#define TEMPI_BTILE(P, W, U, WHOLE, DIR, NT)                                   \
+  copy_tile<P, W, U, WHOLE, DIR, nt_stores(NT, DIR), nt_loads(NT, DIR)>(p, l,  \
+                                                                        nt);   \
+  break;
+#define TEMPI_BCASE(I, P, W, U, NT)                                            \
   case 4 * I + 0:                                                              \
-    copy_tile<P, W, U, false, 0, NTS, NTL>(p, l, nt);                          \
-    break;                                                                     \
+    TEMPI_BTILE(P, W, U, false, 0, NT)                                         \
   case 4 * I + 1:                                                              \
-    copy_tile<P, W, U, false, 1, NTS, NTL>(p, l, nt);                          \
-    break;                                                                     \
+    TEMPI_BTILE(P, W, U, false, 1, NT)                                         \
   case 4 * I + 2:                                                              \
-    copy_tile<P, W, U, true, 0, NTS, NTL>(p, l, nt);                           \
-    break;                                                                     \
+    TEMPI_BTILE(P, W, U, true, 0, NT)                                          \
   case 4 * I + 3:                                                              \
-    copy_tile<P, W, U, true, 1, NTS, NTL>(p, l, nt);                           \
-    break;
+    TEMPI_BTILE(P, W, U, true, 1, NT)
     TEMPI_VARIANTS(TEMPI_BCASE)
 #undef TEMPI_BCASE
+#undef TEMPI_BTILE
   default:
     break;
   }
@@ -526,6 +527,7 @@ TEMPI_EXPORT int tempi_batch_create(const tempi_batch_request *reqs, int64_t n,
   }
   if (method == TEMPI_SELECT_DEFAULT) {
     saturated_batch_policy(reqs, where, &rs);
+    //stream_batch(reqs, where, &rs);
   }
   for (size_t k = 0; k < rs.size(); ++k) {
     b->variants[(size_t)where[k]] = rs[k].variant;
@@ -836,6 +838,7 @@ TEMPI_EXPORT int tempi_batch_run_noalloc(const tempi_batch_request *reqs,
   if (rs.empty()) {
     return TEMPI_SUCCESS;
   }
+  //stream_batch(reqs, where, &rs);
   BatchPlan pl;
   if ((err = plan_batch(rs, device_cu_count(), &pl))) {
     return err;

@@ -293,28 +293,39 @@ __device__ __forceinline__ void copy_units(const KParams &p, uint32_t first,
 
 constexpr int kBlock = 256;
 
-// The variant list, as X(index, P, W, U, NTS, NTL): P lanes per row, W-byte
-// words, U words per lane per unit, nontemporal stores / loads.
+// The variant list, as X(index, P, W, U, NT): P lanes per row, W-byte words,
+// U words per lane per unit, and which side's accesses are nontemporal:
+// kPlain none, kLoads the loads, kStrided those of the strided side (a pack's
+// loads, an unpack's stores).
+enum Nontemporal { kPlain, kLoads, kStrided };
 #define TEMPI_VARIANTS(X)                                                      \
-  X(0, 64, 16, 1, false, false) /* long rows, 1 KiB per wavefront unit */     \
-  X(1, 64, 16, 4, false, false) /* long rows, 4 KiB per unit           */     \
-  X(2, 64, 16, 4, true, false)  /* as 1, nontemporal stores            */     \
-  X(3, 32, 16, 2, false, false) /* rows around 512 B - 1 KiB           */     \
-  X(4, 16, 16, 2, false, false) /* rows around 256 - 512 B             */     \
-  X(5, 8, 16, 2, false, false)  /* rows around 128 - 256 B             */     \
-  X(6, 4, 16, 2, false, false)  /* rows around 64 - 128 B              */     \
-  X(7, 1, 16, 4, false, false)  /* lane per row, 16-B words            */     \
-  X(8, 1, 8, 4, false, false)   /* lane per row, 8-B words             */     \
-  X(9, 1, 4, 4, false, false)   /* lane per row, 4-B words             */     \
-  X(10, 16, 4, 4, false, false) /* 4-B words across 16 lanes           */     \
-  X(11, 1, 1, 16, false, false) /* lane per row, bytes                 */     \
-  X(12, 1, 12, 2, false, false) /* lane per row, 12-B words (3 floats) */     \
-  X(13, 64, 16, 4, false, true) /* as 1, nontemporal loads             */     \
-  X(14, 32, 16, 2, false, true) /* as 3, nontemporal loads             */     \
-  X(15, 16, 16, 2, false, true) /* as 4, nontemporal loads             */     \
-  X(16, 8, 16, 2, false, true)  /* as 5, nontemporal loads             */     \
-  X(17, 4, 16, 2, false, true)  /* as 6, nontemporal loads             */     \
-  X(18, 1, 8, 4, false, true)   /* as 8, nontemporal loads             */
+  X(0, 8, 16, 2, kStrided)  /* as 5, strided side nontemporal      */          \
+  X(1, 64, 16, 4, kPlain)   /* long rows, 4 KiB per unit           */          \
+  X(2, 32, 16, 2, kStrided) /* long rows, strided side nontemporal */          \
+  X(3, 32, 16, 2, kLoads)   /* long rows, nontemporal loads        */          \
+  X(4, 16, 16, 2, kPlain)   /* rows around 256 B - 1 KiB           */          \
+  X(5, 8, 16, 2, kPlain)    /* rows around 128 - 256 B             */          \
+  X(6, 4, 16, 2, kPlain)    /* rows around 64 - 128 B              */          \
+  X(7, 1, 16, 4, kPlain)    /* lane per row, 16-B words            */          \
+  X(8, 1, 8, 4, kPlain)     /* lane per row, 8-B words             */          \
+  X(9, 1, 4, 4, kPlain)     /* lane per row, 4-B words             */          \
+  X(10, 16, 4, 4, kPlain)   /* 4-B words across 16 lanes           */          \
+  X(11, 1, 1, 16, kPlain)   /* lane per row, bytes                 */          \
+  X(12, 1, 12, 2, kPlain)   /* lane per row, 12-B words (3 floats) */          \
+  X(13, 8, 16, 2, kLoads)   /* as 5, nontemporal loads             */          \
+  X(14, 4, 16, 2, kStrided) /* as 6, strided side nontemporal      */          \
+  X(15, 4, 16, 2, kLoads)   /* as 6, nontemporal loads             */          \
+  X(16, 1, 12, 2, kLoads)   /* as 12, nontemporal loads            */          \
+  X(17, 4, 8, 1, kLoads)    /* rows of 8 - 32 B, nontemporal loads */          \
+  X(18, 1, 8, 4, kLoads)    /* as 8, nontemporal loads             */
+
+// nontemporal stores / loads of a variant's kernel in direction DIR
+constexpr bool nt_stores(Nontemporal nt, int dir) {
+  return nt == kStrided && dir == 1;
+}
+constexpr bool nt_loads(Nontemporal nt, int dir) {
+  return nt == kLoads || (nt == kStrided && dir == 0);
+}
 
 // Work units of one launch stay below 2^31.  The kernels index units with
 // 32-bit counters that step by at most (grid * groups * units in flight)

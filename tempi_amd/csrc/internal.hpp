@@ -219,8 +219,8 @@ int make_geom(const tempi_strided_block &sb, int64_t count, Geom *g);
 
 struct VariantDesc {
   int P, W, U;
-  int NTS; // nontemporal stores
-  int NTL; // nontemporal loads
+  int NTS; // nontemporal stores (of unpacks)
+  int NTL; // nontemporal loads (with NTS: of packs only)
 };
 extern const VariantDesc kVariants[];
 extern const int kNumVariants;
@@ -257,6 +257,11 @@ int wait_library_stream();
 // closed-form variant rule (the "plain heuristic")
 int heuristic_variant(const Geom &g, const char *strided, const char *packed,
                       int dir);
+// bytes of the 128-B lines a copy's strided side touches, and the variant
+// for a copy that touches that much where `variant` was picked
+int64_t touched_bytes(const Geom &g);
+int streamed_variant(int variant, const Geom &g, const char *strided, int dir,
+                     int64_t touched);
 
 // the variant for a copy that runs alone and is bound by its launch; -1: it
 // is too large for that

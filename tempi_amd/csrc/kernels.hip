@@ -34,6 +34,7 @@
 
 #include <algorithm>
 #include <chrono>
+#include <cmath>
 
 namespace tempi {
 
@@ -112,22 +113,23 @@ __global__ void __launch_bounds__(kBlock) k_strided_copy(KParams p) {
 // variant table
 // ---------------------------------------------------------------------------
 
-#define TEMPI_VDESC(I, P, W, U, NTS, NTL) {P, W, U, NTS ? 1 : 0, NTL ? 1 : 0},
+#define TEMPI_VDESC(I, P, W, U, NT) {P, W, U, nt_stores(NT, 1), nt_loads(NT, 0)},
 const VariantDesc kVariants[] = {TEMPI_VARIANTS(TEMPI_VDESC)};
 #undef TEMPI_VDESC
 const int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 
 typedef void (*KernelFn)(KParams);
 
-#define TEMPI_KROW(I, P, W, U, NTS, NTL)                                         \
-  {{k_strided_copy<P, W, U, false, 0, NTS, NTL>,                               \
-    k_strided_copy<P, W, U, false, 1, NTS, NTL>},                              \
-   {k_strided_copy<P, W, U, true, 0, NTS, NTL>,                                \
-    k_strided_copy<P, W, U, true, 1, NTS, NTL>}},
+#define TEMPI_KFN(P, W, U, WHOLE, DIR, NT)                                     \
+  k_strided_copy<P, W, U, WHOLE, DIR, nt_stores(NT, DIR), nt_loads(NT, DIR)>
+#define TEMPI_KROW(I, P, W, U, NT)                                             \
+  {{TEMPI_KFN(P, W, U, false, 0, NT), TEMPI_KFN(P, W, U, false, 1, NT)},       \
+   {TEMPI_KFN(P, W, U, true, 0, NT), TEMPI_KFN(P, W, U, true, 1, NT)}},
 
 // [variant][whole rows][dir]
 static const KernelFn kKernels[][2][2] = {TEMPI_VARIANTS(TEMPI_KROW)};
 #undef TEMPI_KROW
+#undef TEMPI_KFN
 static_assert(sizeof(kKernels) / sizeof(kKernels[0]) ==
                   sizeof(kVariants) / sizeof(kVariants[0]),
               "kernel and variant tables differ");
@@ -213,45 +215,126 @@ static int max_aligned_word(const Geom &g, const char *strided,
   return 1;
 }
 
+// Bytes of the strided side's 128-B lines: a row moves the lines it touches,
+// about L + 127 bytes, unless its neighbours share them.
+int64_t touched_bytes(const Geom &g) {
+  if (g.nrd == 0) {
+    return g.L;
+  }
+  const double L = (double)g.L, apart = std::abs((double)g.str[0]);
+  const double bytes =
+      (double)g.rows * std::min(L + 127, std::max(L, apart));
+  return bytes < 1e18 ? (int64_t)bytes : (int64_t)1e18;
+}
+
+// Copies whose strided side touches this much are streamed (below).
+constexpr int64_t kStreamBytes = 64ll << 20;
+constexpr int64_t kInfinityCache = 256ll << 20;
+
+// the variant nearest to a nontemporal one whose accesses are all cached
+static int plain_variant(int v) {
+  switch (v) {
+  case 0:
+  case 13:
+    return 5;
+  case 2:
+  case 3:
+    return 4;
+  case 14:
+  case 15:
+    return 6;
+  case 16:
+    return 12;
+  case 17:
+  case 18:
+    return 8;
+  default:
+    return v;
+  }
+}
+
+// The variant for a copy whose strided side touches `touched` bytes, where
+// `variant` was picked among the cached ones: itself while that is small
+// against the Infinity Cache (256 MiB), else the nontemporal one for the row
+// length.  A program touches the strided side once per pass -- a pack's
+// source and an unpack's destination are a grid it goes on to compute on --
+// while the packed bytes go to the next kernel or to the network, so the
+// strided side is kept out of the caches and the packed stores stay in them.
+// Pack then unpack of the same bytes, three buffer sets in turn (MI355X, us
+// per pass):
+//   4 Mi rows of 64 B at 192 B         cached 307, loads + strided stores 231
+//   256 Ki rows of 1 KiB at 1072 B     cached 231, loads + strided stores 176
+//   512 Ki rows of 64 B at 1777 B      cached 80, loads + strided stores 64,
+//                                      loads on both sides 45
+//   640 Ki rows of 12 B at 1001 B      cached 61, loads + strided stores 88,
+//                                      loads on both sides 38
+// Below 64 MiB of lines cached accesses are as fast or up to 10 % faster.
+//
+// A nontemporal store that covers part of a 64-B sector goes to memory by
+// itself, where a cached one waits in the Infinity Cache for its neighbours:
+// short rows never take them, rows that cut sectors only when their lines
+// could not stay cached anyway.  Then the packed stream is read nontemporal
+// instead, which leaves the cache to those lines.  And a line that two
+// instructions read nontemporal is fetched twice: rows must be covered by
+// one access of a group, or be long.  (600 000 rows of 100 B at 1138 B, 96 B
+// in 16-B words and a 4-B tail, one buffer set: cached 68 us per pass, loads
+// on both sides 86; 24-B rows as three 8-B words of a lane: 93, as one word
+// of three lanes: 64.)
+int streamed_variant(int variant, const Geom &g, const char *strided, int dir,
+                     int64_t touched) {
+  const int plain = plain_variant(variant);
+  if (touched < kStreamBytes) {
+    return plain;
+  }
+  // the packed address does not matter: the strided one stands in for it
+  const bool sectors = geom_aligned(g, strided, strided + g.start, 64);
+  const bool stores =
+      dir == TEMPI_DIR_UNPACK && g.L >= 16 &&
+      (touched > kInfinityCache || (sectors && touched >= kInfinityCache / 2));
+  if (g.L > 512 || (g.L % 16 == 0 && g.L > 128)) {
+    return stores ? 2 : 3;
+  }
+  if (g.L % 16 == 0) {
+    return g.L > 64 ? (stores ? 0 : 13) : (stores ? 14 : 15);
+  }
+  if (g.L == 12) {
+    return 16;
+  }
+  if (g.L % 8 == 0 && g.L <= 32) {
+    return 17;
+  }
+  if (g.L == 1 || g.L == 2 || g.L == 4) {
+    return 18;
+  }
+  return plain;
+}
+
 int heuristic_variant(const Geom &g, const char *strided, const char *packed,
                       int dir) {
-  (void)dir;
   const int64_t L = g.L;
-  const int64_t bytes = L * g.rows;
-  // Copies this large are read from HBM: nontemporal loads let their line
-  // fills go first from the caches, ahead of the lines being written.
-  const bool big = bytes >= (8ll << 20);
-  if (L >= 1024) {
-    // one long run: nontemporal stores
-    if (g.rows == 1) {
-      return big ? 2 : 0;
+  int v = 11;
+  if (L >= 2048) {
+    v = 1;
+  } else if (L >= 256) {
+    v = 4;
+  } else if (L >= 128) {
+    v = 5;
+  } else if (L >= 64) {
+    v = 6;
+  } else {
+    const int Wa = max_aligned_word(g, strided, packed);
+    if (Wa >= 16) {
+      v = 7;
+    } else if (Wa == 8) {
+      v = 8;
+    } else if (Wa == 4) {
+      // rows of 3 or 6 dwords move as 12-B words
+      v = (L % 12 == 0) ? 12 : 9;
+    } else if (L >= 16) {
+      v = 7;
     }
-    return big ? 13 : 0;
   }
-  if (L >= 512) {
-    return big ? 14 : 3;
-  }
-  if (L >= 256) {
-    return big ? 15 : 4;
-  }
-  if (L >= 128) {
-    return big ? 16 : 5;
-  }
-  if (L >= 64) {
-    return big ? 17 : 6;
-  }
-  const int Wa = max_aligned_word(g, strided, packed);
-  if (Wa >= 16) {
-    return 7;
-  }
-  if (Wa == 8) {
-    return big ? 18 : 8;
-  }
-  if (Wa == 4) {
-    // rows of 3 or 6 dwords move as 12-B words
-    return (L % 12 == 0) ? 12 : 9;
-  }
-  return L >= 16 ? 7 : 11;
+  return streamed_variant(v, g, strided, dir, touched_bytes(g));
 }
 
 // Launched back to back, all variants move a copy of up to 1 MiB at the
@@ -812,7 +895,7 @@ void emulate_unit(const KParams &p, uint32_t u) {
 }
 
 typedef void (*EmulateFn)(const KParams &, uint32_t);
-#define TEMPI_EROW(I, P, W, U, NTS, NTL)                                         \
+#define TEMPI_EROW(I, P, W, U, NT)                                             \
   {{emulate_unit<P, W, U, false, 0>, emulate_unit<P, W, U, false, 1>},          \
    {emulate_unit<P, W, U, true, 0>, emulate_unit<P, W, U, true, 1>}},
 const EmulateFn kEmulate[][2][2] = {TEMPI_VARIANTS(TEMPI_EROW)};

@@ -37,7 +37,7 @@ namespace tempi {
 
 namespace {
 
-#define TEMPI_COUNT_V(I, P, W, U, NTS, NTL) +1
+#define TEMPI_COUNT_V(I, P, W, U, NT) +1
 constexpr int kOut = 0 TEMPI_VARIANTS(TEMPI_COUNT_V);
 #undef TEMPI_COUNT_V
 constexpr int kIn = 16, kH1 = 64, kH2 = 64;
