@@ -230,7 +230,7 @@ int tempi_autotune(const tempi_strided_block *sb, int64_t incount,
    arithmetic the library uses for (variant, grid cap) -- with the kernels'
    own address code -- and records the bytes each launch would load and
    store, without touching memory (the addresses are numbers only).
-   `max_blocks` is a workgroup cap (0: the default, 16 per CU) and
+   `max_blocks` is a workgroup cap (0: the default, 256 per CU) and
    `cu_count` the CU count it assumes.  Copies of more than `unit_limit`
    work units report only the launch plan (emulated = 0). */
 typedef struct tempi_copy_emulation {

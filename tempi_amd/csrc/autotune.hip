@@ -18,7 +18,7 @@
 
 namespace tempi {
 
-// multiples of the CU count; 0 = the launch code's default (16 per CU)
+// multiples of the CU count; 0 = the launch code's default (256 per CU)
 const int kGridCaps[] = {0, 2, 4, 8, 32};
 
 // Copies of at least kColdBytes packed bytes are timed one launch at a time,

@@ -329,7 +329,7 @@ constexpr bool nt_loads(Nontemporal nt, int dir) {
 
 // Work units of one launch stay below 2^31.  The kernels index units with
 // 32-bit counters that step by at most (grid * groups * units in flight)
-// < 2^24 past the last unit, so no index wraps; launch_copy splits a larger
+// < 2^28 past the last unit, so no index wraps; launch_copy splits a larger
 // copy along its outer row dimensions.
 constexpr int64_t kMaxUnits = 1ll << 31;
 
