@@ -174,7 +174,8 @@ int tempi_variant_info_get(int variant, tempi_variant_info *info);
 
 /* Variant the library would use for this copy.  Under the default policy a
    copy of at most 1 MiB (128 KiB in rows under 64 B) takes a closed-form
-   choice: it is bound by its launch, not by the kernel.  A copy of 64 MiB or
+   choice: it is bound by its launch, not by the kernel.  So does one of
+   512 KiB or more whose packed side is host memory: the link bounds it.  A copy of 64 MiB or
    more is settled on its first run: the model's three best variants and the
    closed-form rule's pick are each timed once, cold, writing a scratch image
    of the destination (never the caller's buffers), and the fastest is kept

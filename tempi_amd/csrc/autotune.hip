@@ -369,6 +369,10 @@ Choice choose(const Geom &g, const char *strided, char *packed, int dir,
       (c.variant = latency_variant(g)) >= 0) {
     return c;
   }
+  if (method == TEMPI_SELECT_DEFAULT && g.host &&
+      (c.variant = link_variant(g, dir)) >= 0) {
+    return c;
+  }
   c.variant = heuristic_variant(g, strided, packed, dir);
   if (method == TEMPI_SELECT_MODEL ||
       (method == TEMPI_SELECT_DEFAULT && model_available())) {

@@ -193,7 +193,8 @@ hipStream_t library_stream(); // valid after ensure_runtime()
 int library_device();          // the device of library_stream()
 int device_cu_count();
 // returns 1 and the device-usable address when the kernels can read/write p
-int device_address(const void *p, void **dev);
+// (*host, when given: it is host memory)
+int device_address(const void *p, void **dev, bool *host = nullptr);
 // true for device memory the host cannot load or store (not host-mapped,
 // not managed)
 bool device_only(const void *p);
@@ -214,6 +215,7 @@ struct Geom {
   int64_t cnt[kMaxRowDims] = {};
   int64_t str[kMaxRowDims] = {};
   int64_t start = 0; // byte offset of row 0 from the strided buffer origin
+  bool host = false; // the packed side is host memory
 };
 int make_geom(const tempi_strided_block &sb, int64_t count, Geom *g);
 
@@ -266,6 +268,9 @@ int streamed_variant(int variant, const Geom &g, const char *strided, int dir,
 // the variant for a copy that runs alone and is bound by its launch; -1: it
 // is too large for that
 int latency_variant(const Geom &g);
+// the variant for a copy that runs alone and whose packed side is host
+// memory; -1: it is too small to be bound by the link
+int link_variant(const Geom &g, int dir);
 
 // a kernel variant and its grid cap (0: the default cap)
 struct Choice {
@@ -427,16 +432,17 @@ struct TraceRange {
   TraceRange &operator=(const TraceRange &) = delete;
 };
 // pack (dir 0) or unpack `count` objects on `stream` with the library's
-// variant choice (variant < 0) or the given one; device addresses
+// variant choice (variant < 0) or the given one; device addresses; `host`:
+// the packed one is host memory
 int run_copy(const tempi_strided_block &sb, int64_t count, const char *strided,
-             char *packed, int dir, int variant, hipStream_t stream);
+             char *packed, bool host, int dir, int variant, hipStream_t stream);
 // run_copy on the library stream with the library's variant, returning when
 // the copy is done (launch_copy_wait)
 int run_copy_wait(const tempi_strided_block &sb, int64_t count,
-                  const char *strided, char *packed, int dir);
+                  const char *strided, char *packed, bool host, int dir);
 // the same without waiting; *seq and *own as for launch_copy_signalled
 int run_copy_signalled(const tempi_strided_block &sb, int64_t count,
-                       const char *strided, char *packed, int dir,
+                       const char *strided, char *packed, bool host, int dir,
                        unsigned long long *seq, bool *own);
 
 // cached staging buffers (pool.cpp): device memory, or pinned host memory

@@ -180,7 +180,8 @@ bool lookup(MPI_Datatype t, Canon *out) { return type_lookup(t, out); }
 // `strided` / `packed` are device addresses of the strided buffer origin and
 // of the first packed byte.
 int run_copy(const tempi_strided_block &sb, int64_t count, const char *strided,
-             char *packed, int dir, int variant, hipStream_t stream) {
+             char *packed, bool host, int dir, int variant,
+             hipStream_t stream) {
   Geom g;
   int err = make_geom(sb, count, &g);
   if (err) {
@@ -189,6 +190,7 @@ int run_copy(const tempi_strided_block &sb, int64_t count, const char *strided,
   if (g.rows == 0) {
     return TEMPI_SUCCESS;
   }
+  g.host = host;
   Choice c;
   if (variant < 0) {
     c = choose(g, strided, packed, dir, env().select, stream,
@@ -201,7 +203,7 @@ int run_copy(const tempi_strided_block &sb, int64_t count, const char *strided,
 
 // run_copy on the library stream, returning when the copy is done
 int run_copy_wait(const tempi_strided_block &sb, int64_t count,
-                         const char *strided, char *packed, int dir) {
+                  const char *strided, char *packed, bool host, int dir) {
   Geom g;
   int err = make_geom(sb, count, &g);
   if (err) {
@@ -210,6 +212,7 @@ int run_copy_wait(const tempi_strided_block &sb, int64_t count,
   if (g.rows == 0) {
     return TEMPI_SUCCESS;
   }
+  g.host = host;
   const Choice c = choose(g, strided, packed, dir, env().select,
                           library_stream(), CopyUse::kNext);
   return launch_copy_wait(g, strided, packed, dir, c.variant, c.max_blocks);
@@ -218,7 +221,7 @@ int run_copy_wait(const tempi_strided_block &sb, int64_t count,
 // run_copy on the library stream without waiting; *seq > 0: the signal to
 // wait for (signal_reached)
 int run_copy_signalled(const tempi_strided_block &sb, int64_t count,
-                       const char *strided, char *packed, int dir,
+                       const char *strided, char *packed, bool host, int dir,
                        unsigned long long *seq, bool *own) {
   *seq = 0;
   *own = false;
@@ -230,6 +233,7 @@ int run_copy_signalled(const tempi_strided_block &sb, int64_t count,
   if (g.rows == 0) {
     return TEMPI_SUCCESS;
   }
+  g.host = host;
   const Choice c = choose(g, strided, packed, dir, env().select,
                           library_stream(), CopyUse::kNext);
   return launch_copy_signalled(g, strided, packed, dir, c.variant,
@@ -245,14 +249,15 @@ struct HostStage {
 
 // MPI_Pack / MPI_Unpack on device-accessible buffers.  `strided` is the
 // device address of the strided buffer; `packed` is the first packed byte,
-// either a device address or, with `host_packed`, pageable host memory the
-// device cannot address: then the kernel reads or writes a pinned host
-// staging buffer through its device mapping (as ONE_SHOT does) and the host
-// copies between it and the caller's memory -- a kernel store across the
-// link plus a host memcpy, where a copy from device memory into pageable
-// memory would go through the runtime's own bounce buffer.
+// either a device address (`host`: of mapped host memory) or, with
+// `host_packed`, pageable host memory the device cannot address: then the
+// kernel reads or writes a pinned host staging buffer through its device
+// mapping (as ONE_SHOT does) and the host copies between it and the caller's
+// memory -- a kernel store across the link plus a host memcpy, where a copy
+// from device memory into pageable memory would go through the runtime's own
+// bounce buffer.
 int pack_or_unpack(const Canon &cn, int count, const char *strided,
-                   char *packed, bool host_packed, int dir) {
+                   char *packed, bool host_packed, bool host, int dir) {
   const int64_t bytes = (int64_t)count * cn.size;
   HostStage stage;
   char *kernel_packed = packed;
@@ -271,7 +276,8 @@ int pack_or_unpack(const Canon &cn, int count, const char *strided,
   }
   // returns once the copy is done (also on failure: the staging buffer is
   // read, or goes back to the pool, only after that)
-  const int err = run_copy_wait(cn.sb, count, strided, kernel_packed, dir);
+  const int err = run_copy_wait(cn.sb, count, strided, kernel_packed,
+                                host || host_packed, dir);
   if (!err && host_packed && dir == TEMPI_DIR_PACK) {
     memcpy(packed, stage.p, (size_t)bytes);
   }
@@ -484,7 +490,8 @@ TEMPI_EXPORT int MPI_Pack(const void *inbuf, int incount, MPI_Datatype datatype,
     ++counters().library_pack_calls;
     return lib.Pack(inbuf, incount, datatype, outbuf, outsize, position, comm);
   }
-  const bool host_packed = !device_address(outbuf, &dout);
+  bool mapped = false;
+  const bool host_packed = !device_address(outbuf, &dout, &mapped);
   const int64_t packed = (int64_t)incount * cn.size;
   if (*position < 0 || (int64_t)*position + packed > (int64_t)outsize) {
     // the reference writes past the end here (pack.cpp:56)
@@ -498,7 +505,8 @@ TEMPI_EXPORT int MPI_Pack(const void *inbuf, int incount, MPI_Datatype datatype,
   char *packed_at =
       static_cast<char *>(host_packed ? outbuf : dout) + *position;
   const int err = pack_or_unpack(cn, incount, static_cast<const char *>(din),
-                                 packed_at, host_packed, TEMPI_DIR_PACK);
+                                 packed_at, host_packed, mapped,
+                                 TEMPI_DIR_PACK);
   if (err) {
     TEMPI_LOG(LOG_ERROR, "MPI_Pack: %s", tempi_last_error());
     MPI_Comm_call_errhandler(comm, MPI_ERR_INTERN);
@@ -533,7 +541,8 @@ TEMPI_EXPORT int MPI_Unpack(const void *inbuf, int insize, int *position,
     return lib.Unpack(inbuf, insize, position, outbuf, outcount, datatype,
                       comm);
   }
-  const bool host_packed = !device_address(inbuf, &din);
+  bool mapped = false;
+  const bool host_packed = !device_address(inbuf, &din, &mapped);
   const int64_t packed = (int64_t)outcount * cn.size;
   if (*position < 0 || (int64_t)*position + packed > (int64_t)insize) {
     MPI_Comm_call_errhandler(comm, MPI_ERR_TRUNCATE);
@@ -548,7 +557,8 @@ TEMPI_EXPORT int MPI_Unpack(const void *inbuf, int insize, int *position,
       static_cast<char *>(host_packed ? const_cast<void *>(inbuf) : din) +
       *position;
   const int err = pack_or_unpack(cn, outcount, static_cast<const char *>(dout),
-                                 packed_at, host_packed, TEMPI_DIR_UNPACK);
+                                 packed_at, host_packed, mapped,
+                                 TEMPI_DIR_UNPACK);
   if (err) {
     TEMPI_LOG(LOG_ERROR, "MPI_Unpack: %s", tempi_last_error());
     MPI_Comm_call_errhandler(comm, MPI_ERR_INTERN);
@@ -655,6 +665,8 @@ TEMPI_EXPORT int tempi_select_variant(const tempi_strided_block *sb,
                    .variant;
     return TEMPI_SUCCESS;
   }
+  void *dp = nullptr;
+  (void)device_address(packed_buf, &dp, &g.host);
   *variant = choose(g, static_cast<const char *>(strided_buf),
                     static_cast<char *>(const_cast<void *>(packed_buf)),
                     direction, method, nullptr, CopyUse::kQuery)
@@ -683,13 +695,14 @@ TEMPI_EXPORT int tempi_pack_sb(const tempi_strided_block *sb,
     return err;
   }
   void *din = nullptr, *dout = nullptr;
+  bool host = false;
   if (packed > 0 &&
-      (!device_address(inbuf, &din) || !device_address(outbuf, &dout))) {
+      (!device_address(inbuf, &din) || !device_address(outbuf, &dout, &host))) {
     return set_error(TEMPI_ERR_ARG, "buffers must be device-accessible");
   }
   hipStream_t s = stream ? static_cast<hipStream_t>(stream) : library_stream();
   err = run_copy(*sb, incount, static_cast<const char *>(din),
-                 static_cast<char *>(dout) + *position, TEMPI_DIR_PACK,
+                 static_cast<char *>(dout) + *position, host, TEMPI_DIR_PACK,
                  variant, s);
   if (err) {
     return err;
@@ -719,13 +732,14 @@ TEMPI_EXPORT int tempi_unpack_sb(const tempi_strided_block *sb,
     return err;
   }
   void *din = nullptr, *dout = nullptr;
+  bool host = false;
   if (packed > 0 &&
-      (!device_address(inbuf, &din) || !device_address(outbuf, &dout))) {
+      (!device_address(inbuf, &din, &host) || !device_address(outbuf, &dout))) {
     return set_error(TEMPI_ERR_ARG, "buffers must be device-accessible");
   }
   hipStream_t s = stream ? static_cast<hipStream_t>(stream) : library_stream();
   err = run_copy(*sb, outcount, static_cast<const char *>(dout),
-                 static_cast<char *>(din) + *position, TEMPI_DIR_UNPACK,
+                 static_cast<char *>(din) + *position, host, TEMPI_DIR_UNPACK,
                  variant, s);
   if (err) {
     return err;

@@ -375,6 +375,27 @@ int latency_variant(const Geom &g) {
   return L % 4 == 0 || L < 16 ? 9 : 7;
 }
 
+// Copies to or from host memory are bound by the link (57 GB/s).  Stores reach
+// it from any variant whose words lie together; loads do only where a
+// wavefront's lanes read apart from each other -- lane per row, or 16 B per
+// lane in dwords -- and not where they read one contiguous KiB, at any grid
+// size.  4 MiB unpacked from mapped memory, us (floor 73.3):
+//   rows of 64 B    variant 9 78, 7 78, 10 77, 6 101, 8 101
+//   rows of 256 B   variant 9 78, 7 78, 4 101, 6 100, 10 103
+//   rows of 4 KiB   variant 9 76, 7 77, 1 98, 4 98, 10 101
+// Over 55 copies of 0.5 to 15 MiB, rows of 1 B to 4 KiB, the selector, which is
+// trained on device memory, unpacked 11.9 % slower than the best variant and
+// packed 1.8 %; this rule 1.3 % and 0.7 %.
+int link_variant(const Geom &g, int dir) {
+  if (g.L * g.rows < 512 << 10) {
+    return -1;
+  }
+  if (dir == TEMPI_DIR_UNPACK) {
+    return 9;
+  }
+  return g.L >= 256 ? 4 : g.L >= 128 ? 5 : g.L >= 32 ? 6 : g.L % 8 ? 9 : 8;
+}
+
 int fill_kparams(const Geom &g, const char *strided, char *packed, int dir,
                  int variant, KParams *pp, bool *whole) {
   const VariantDesc &v = kVariants[variant];

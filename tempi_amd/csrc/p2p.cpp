@@ -208,15 +208,16 @@ struct Staging {
   void *wire() const { return method == TEMPI_METHOD_DEVICE ? dev : host; }
   // where the kernels write packed bytes / read them
   char *kernel_side() const {
-    return static_cast<char *>(method == TEMPI_METHOD_ONESHOT ? host_dev : dev);
+    return static_cast<char *>(kernel_host() ? host_dev : dev);
   }
+  bool kernel_host() const { return method == TEMPI_METHOD_ONESHOT; }
 };
 
 // enqueue pack (+ copy to host) of `count` objects into the staging buffer
 int enqueue_pack(const Canon &cn, int count, const void *ubuf_dev, Staging &st,
                  hipStream_t s) {
   int err = run_copy(cn.sb, count, static_cast<const char *>(ubuf_dev),
-                     st.kernel_side(), TEMPI_DIR_PACK, -1, s);
+                     st.kernel_side(), st.kernel_host(), TEMPI_DIR_PACK, -1, s);
   if (!err && st.method == TEMPI_METHOD_STAGED) {
     TEMPI_HIP_CHECK(hipMemcpyAsync(st.host, st.dev, (size_t)st.bytes,
                                    hipMemcpyDeviceToHost, s));
@@ -232,7 +233,7 @@ int enqueue_unpack(const Canon &cn, int count, void *ubuf_dev, Staging &st,
                                    hipMemcpyHostToDevice, s));
   }
   return run_copy(cn.sb, count, static_cast<const char *>(ubuf_dev),
-                  st.kernel_side(), TEMPI_DIR_UNPACK, -1, s);
+                  st.kernel_side(), st.kernel_host(), TEMPI_DIR_UNPACK, -1, s);
 }
 
 int mpi_error_of(int tempi_err) {
@@ -383,7 +384,7 @@ public:
     int err = stg_.acquire(method, bytes_);
     if (!err && method != TEMPI_METHOD_STAGED) {
       err = run_copy_signalled(cn.sb, count, static_cast<const char *>(ubuf_dev),
-                               stg_.kernel_side(), TEMPI_DIR_PACK, &seq_, &own_);
+                               stg_.kernel_side(), stg_.kernel_host(), TEMPI_DIR_PACK, &seq_, &own_);
     } else if (!err) {
       err = enqueue_pack(cn, count, ubuf_dev, stg_, s);
       seq_ = err ? 0 : signal_stream();
@@ -464,7 +465,7 @@ class IrecvOp : public AsyncOp {
     int err = TEMPI_SUCCESS;
     if (stg_.method != TEMPI_METHOD_STAGED) {
       err = run_copy_signalled(cn_.sb, n, static_cast<const char *>(ubuf_dev_),
-                               stg_.kernel_side(), TEMPI_DIR_UNPACK, &seq_,
+                               stg_.kernel_side(), stg_.kernel_host(), TEMPI_DIR_UNPACK, &seq_,
                                &own_);
     } else {
       err = enqueue_unpack(cn_, n, ubuf_dev_, stg_, (int64_t)n * cn_.size, s);
@@ -814,7 +815,7 @@ TEMPI_EXPORT int MPI_Send(const void *buf, int count, MPI_Datatype datatype,
   if (!terr && method != TEMPI_METHOD_STAGED) {
     // the pack is all there is to wait for
     terr = run_copy_wait(cn.sb, count, static_cast<const char *>(dev),
-                         st.kernel_side(), TEMPI_DIR_PACK);
+                         st.kernel_side(), st.kernel_host(), TEMPI_DIR_PACK);
   } else if (!terr) {
     terr = enqueue_pack(cn, count, dev, st, s);
     if (!terr) {
@@ -888,7 +889,7 @@ TEMPI_EXPORT int MPI_Recv(void *buf, int count, MPI_Datatype datatype,
     int terr = TEMPI_SUCCESS;
     if (method != TEMPI_METHOD_STAGED) {
       terr = run_copy_wait(cn.sb, n, static_cast<const char *>(dev),
-                           st.kernel_side(), TEMPI_DIR_UNPACK);
+                           st.kernel_side(), st.kernel_host(), TEMPI_DIR_UNPACK);
     } else {
       terr = enqueue_unpack(cn, n, dev, st, (int64_t)n * cn.size, s);
       if (!terr) {

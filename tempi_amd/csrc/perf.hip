@@ -769,8 +769,9 @@ int measure_table(int table, const Sampling &sampling, Table *out) {
           tempi_free_host_mapped(p);
         }
       });
+  bool packed_host = false;
   void *packed_dev = nullptr;
-  if (!device_address(packed, &packed_dev)) {
+  if (!device_address(packed, &packed_dev, &packed_host)) {
     return set_error(TEMPI_ERR_HIP, "no device address for the packed buffer");
   }
   hipStream_t s = library_stream();
@@ -796,6 +797,7 @@ int measure_table(int table, const Sampling &sampling, Table *out) {
       }
       const char *sp = static_cast<const char *>(strided.p);
       char *pp = static_cast<char *>(packed_dev);
+      g.host = packed_host;
       const Choice ch = choose(g, sp, pp, dir, env().select, s,
                                CopyUse::kNext);
       IidTime r;

@@ -130,8 +130,11 @@ int library_device() { return rt().device; }
 
 int device_cu_count() { return rt().cus > 0 ? rt().cus : 256; }
 
-int device_address(const void *p, void **dev) {
+int device_address(const void *p, void **dev, bool *host) {
   *dev = nullptr;
+  if (host) {
+    *host = false;
+  }
   if (!p || !have_device()) {
     return 0;
   }
@@ -150,6 +153,9 @@ int device_address(const void *p, void **dev) {
   case hipMemoryTypeHost:
     if (!a.devicePointer) {
       return 0;
+    }
+    if (host) {
+      *host = true;
     }
     if (a.hostPointer && a.hostPointer != p) {
       // attributes describe the allocation base
