@@ -51,14 +51,13 @@ FastDiv make_fastdiv(uint32_t d) {
   return f;
 }
 
-// Where signalled copies count their finished workgroups and report to the
-// host; set once by the host (signal_ready) before the first signalled
-// launch.
+// Where a signalled copy counts its finished workgroups and reports to the
+// host (kernel arguments: read with the copy's own, not through a pointer
+// after it).
 struct SignalSlots {
   uint32_t *counter; // finished workgroups of the running launch
   uint32_t *flag;    // number of the last completed signal, in pinned host memory
 };
-static __device__ SignalSlots g_signal_slots;
 
 // The end of a launch with p.signal set, run by every thread of the
 // workgroup: the workgroup's stores are released at system scope (the
@@ -66,27 +65,31 @@ static __device__ SignalSlots g_signal_slots;
 // thread 0's release, scopes composing), then counted.  The launch's last
 // workgroup resets the counter for the next signalled launch -- launches on
 // the library stream never overlap -- and stores the launch's number to the
-// host's flag.  The count itself is relaxed: the fences before and after it
-// order it, and an ordered one would write the L2 back a second time per
-// workgroup (128 workgroups of 16 KiB, launch to flag: 11.5 -> 10.7 us).
-__device__ __forceinline__ void signal_done(const KParams &p) {
+// host's flag; a workgroup on its own has nothing to count.  The count itself
+// is relaxed: the fences before and after it order it, and an ordered one
+// would write the L2 back a second time per workgroup (128 workgroups of
+// 16 KiB, launch to flag: 11.5 -> 10.7 us).
+__device__ __forceinline__ void signal_done(const KParams &p,
+                                            const SignalSlots &s) {
   if (!p.signal) {
     return;
   }
-  const SignalSlots s = g_signal_slots;
   __syncthreads();
   if (threadIdx.x == 0) {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
-    const uint32_t done = __hip_atomic_fetch_add(s.counter, 1u, __ATOMIC_RELAXED,
-                                                 __HIP_MEMORY_SCOPE_AGENT) +
-                          1u;
-    if (done == gridDim.x) {
+    if (gridDim.x > 1) {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "");
+      if (__hip_atomic_fetch_add(s.counter, 1u, __ATOMIC_RELAXED,
+                                 __HIP_MEMORY_SCOPE_AGENT) +
+              1u !=
+          gridDim.x) {
+        return;
+      }
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "");
       __hip_atomic_store(s.counter, 0u, __ATOMIC_RELAXED,
                          __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(s.flag, p.signal, __ATOMIC_RELEASE,
-                         __HIP_MEMORY_SCOPE_SYSTEM);
     }
+    __hip_atomic_store(s.flag, p.signal, __ATOMIC_RELEASE,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 
@@ -97,7 +100,8 @@ __global__ void k_signal(uint32_t *flag, uint32_t number) {
 }
 
 template <int P, int W, int U, bool WHOLE, int DIR, bool NTS, bool NTL>
-__global__ void __launch_bounds__(kBlock) k_strided_copy(KParams p) {
+__global__ void __launch_bounds__(kBlock)
+    k_strided_copy(KParams p, SignalSlots slots) {
   constexpr uint32_t GROUPS = kBlock / P;
   constexpr uint32_t K = units_in_flight(U);
   const uint32_t lane = threadIdx.x % P;
@@ -106,7 +110,7 @@ __global__ void __launch_bounds__(kBlock) k_strided_copy(KParams p) {
        u += step * K) {
     copy_units<P, W, U, WHOLE, DIR, NTS, NTL>(p, u, step, p.units, lane);
   }
-  signal_done(p);
+  signal_done(p, slots);
 }
 
 // ---------------------------------------------------------------------------
@@ -118,7 +122,7 @@ const VariantDesc kVariants[] = {TEMPI_VARIANTS(TEMPI_VDESC)};
 #undef TEMPI_VDESC
 const int kNumVariants = sizeof(kVariants) / sizeof(kVariants[0]);
 
-typedef void (*KernelFn)(KParams);
+typedef void (*KernelFn)(KParams, SignalSlots);
 
 #define TEMPI_KFN(P, W, U, WHOLE, DIR, NT)                                     \
   k_strided_copy<P, W, U, WHOLE, DIR, nt_stores(NT, DIR), nt_loads(NT, DIR)>
@@ -535,7 +539,8 @@ static int for_each_launch(const Geom &g, const char *strided, char *packed,
 // caller holds the signal's lock).
 static int launch_one(const Geom &g, const char *strided, char *packed,
                       int dir, int variant, hipStream_t stream,
-                      int max_blocks, uint32_t signal = 0) {
+                      int max_blocks, uint32_t signal = 0,
+                      SignalSlots slots = {}) {
   KParams p;
   bool whole = false;
   int err = fill_kparams(g, strided, packed, dir, variant, &p, &whole);
@@ -545,7 +550,7 @@ static int launch_one(const Geom &g, const char *strided, char *packed,
   const int64_t blocks = grid_of(variant, p.units, max_blocks, device_cu_count());
   KernelFn fn = kKernels[variant][whole ? 1 : 0][dir];
   p.signal = signal;
-  void *args[] = {&p};
+  void *args[] = {&p, &slots};
   TEMPI_HIP_CHECK(hipLaunchKernel(reinterpret_cast<const void *>(fn),
                                   dim3((unsigned)blocks), dim3(kBlock), args,
                                   0, stream));
@@ -609,9 +614,8 @@ constexpr int64_t kSignalMaxBlocks = 128;
 struct SignalState {
   std::mutex mu; // held from a signal's number to its launch
   bool tried = false;
-  uint32_t *counter = nullptr;  // device memory
-  uint32_t *flag = nullptr;     // pinned host memory
-  uint32_t *flag_dev = nullptr; // its device address
+  SignalSlots slots{};       // device addresses: device memory, the flag
+  uint32_t *flag = nullptr;  // pinned host memory
   unsigned long long issued = 0; // signals so far
   // set after a signalled wait fails: the counter may no longer match the
   // launches, so later copies wait on the stream
@@ -636,16 +640,15 @@ bool flag_at(const SignalState &st, unsigned long long seq) {
                    (uint32_t)seq) >= 0;
 }
 
-// Counter and flag, allocated and published to the kernels once, on the
-// library stream's device (the state's lock held); false when they cannot be.
+// Counter and flag, allocated once, on the library stream's device (the
+// state's lock held); false when they cannot be.
 bool signal_ready(SignalState &st) {
   if (st.tried) {
     return st.flag != nullptr && !st.off.load(std::memory_order_relaxed);
   }
   st.tried = true;
-  // the zeroed counter and the published slots are in place before the
-  // first signalled launch: both go through the library stream (which does
-  // not wait for the null stream), and it is drained here
+  // the counter is zeroed on the library stream (which does not wait for the
+  // null stream) before the first signalled launch
   hipStream_t s = library_stream();
   void *c = nullptr, *f = nullptr, *fd = nullptr;
   bool ok = hipSuccess == hipMalloc(&c, 256) &&
@@ -655,12 +658,7 @@ bool signal_ready(SignalState &st) {
             hipSuccess == hipHostGetDevicePointer(&fd, f, 0);
   if (ok) {
     __atomic_store_n(static_cast<uint32_t *>(f), 0u, __ATOMIC_RELEASE);
-    const SignalSlots slots{static_cast<uint32_t *>(c),
-                            static_cast<uint32_t *>(fd)};
-    ok = hipSuccess == hipMemcpyToSymbolAsync(HIP_SYMBOL(g_signal_slots), &slots,
-                                              sizeof slots, 0,
-                                              hipMemcpyHostToDevice, s) &&
-         hipSuccess == hipStreamSynchronize(s);
+    ok = hipSuccess == hipStreamSynchronize(s);
   }
   if (!ok) {
     (void)hipGetLastError();
@@ -673,8 +671,7 @@ bool signal_ready(SignalState &st) {
     TEMPI_LOG(LOG_WARN, "no completion signal: synchronous copies wait on the stream");
     return false;
   }
-  st.counter = static_cast<uint32_t *>(c);
-  st.flag_dev = static_cast<uint32_t *>(fd);
+  st.slots = SignalSlots{static_cast<uint32_t *>(c), static_cast<uint32_t *>(fd)};
   st.flag = static_cast<uint32_t *>(f);
   return true;
 }
@@ -747,7 +744,7 @@ unsigned long long signal_stream() {
   }
   const unsigned long long n = next_signal(st);
   hipLaunchKernelGGL(k_signal, dim3(1), dim3(1), 0, library_stream(),
-                     st.flag_dev, (uint32_t)n);
+                     st.slots.flag, (uint32_t)n);
   if (hipSuccess != hipGetLastError()) {
     return 0;
   }
@@ -772,7 +769,7 @@ int launch_copy_signalled(const Geom &g, const char *strided, char *packed,
     if (signal_ready(st)) {
       const unsigned long long n = next_signal(st);
       const int err = launch_one(g, strided, packed, dir, variant, s,
-                                 max_blocks, (uint32_t)n);
+                                 max_blocks, (uint32_t)n, st.slots);
       if (!err) {
         *seq = st.issued = n;
         *own = true;
