@@ -364,7 +364,8 @@ int plan_tables(const std::vector<Req> &rs, BatchPlan *pl) {
   // workgroups per CU that looped over them let neighbouring tiles drift
   // apart: halo batches (below) 276 -> 257 us, the random requests 4.51 ->
   // 3.81 ms.
-  constexpr int64_t cap = 1 << 30;
+  // (A launch has fewer than 2^32 threads: beyond 2^23 tiles the grid loops.)
+  constexpr int64_t cap = 1 << 23;
   if (!items.empty() && items.size() <= (size_t)kSmallItems) {
     // tile index in the kernel arguments; only the parameters go to the
     // device table
@@ -464,7 +465,7 @@ int resolve_requests(const tempi_batch_request *reqs, int64_t n, Pick &&pick,
                        (long long)i);
     }
     void *ds = nullptr, *dp = nullptr;
-    if (!device_address(r.strided, &ds) || !device_address(r.packed, &dp)) {
+    if (!device_address(r.strided, &ds) || !device_address(r.packed, &dp, &q.g.host)) {
       return set_error(TEMPI_ERR_ARG,
                        "request %lld: buffers must be device-accessible",
                        (long long)i);
@@ -545,35 +546,89 @@ uint64_t tiles_of(const Req &q) {
   return (units + per_tile - 1) / per_tile;
 }
 
-// The default policy's batch rule.  The learned selector ranks a copy's
-// variants by the time of the copy alone, where a copy under a megabyte is
-// latency-bound and variants that split it into more tiles win.  In a batch
-// with more tiles than the grid runs at once, throughput decides instead:
-// on MI355X the 1 664-request halo batch (all requests under 1 MiB) packed in
-// 129 us with the closed-form rule's variants against 139 us with the
-// selector's, and unpacked in 174 us against 267 us, while the 4 096 random
-// requests (up to 16 MiB) packed in 8.6 ms with the selector's against 9.2 ms.
-// So in a batch that saturates the grid, requests under 1 MiB whose variant
-// was left to the library take the rule; larger requests, and small batches
-// (the headline's three faces: 9.26 us with the selector's picks against
-// 9.91 us with the rule's), keep the selector's.
-void saturated_batch_policy(const tempi_batch_request *reqs,
-                            const std::vector<int64_t> &where,
-                            std::vector<Req> *rs) {
+// The default policy's rule for batches with more tiles than the grid runs at
+// once.  The learned selector ranks a copy's variants by the time of the copy
+// alone; among other requests what counts is how many bytes a workgroup keeps
+// in flight, so the rule takes the variant whose lanes all have a word to
+// move and which moves most rows per pass.  Rows under 16 B take the 12-B
+// words' kernel whatever their length: a row is one unit of one or two
+// accesses there and a lane has two rows in flight, where the other
+// lane-per-row kernels hold four words of one row, most of which a short row
+// does not have.  Packs of rows of 24-47 B take four lanes of 8 B to a row,
+// and those and packs of rows over 512 B read nontemporal: the lines of a
+// halo's long rows are read once, and leave the caches to those its short
+// rows share.  Unpacks gain or lose by nontemporal loads with the size of
+// the batch (64 subdomains of 96^3, rows of 8 B, 78 -> 57 us, of 12 B 92 ->
+// 111) and do without.  Random requests of 4 KiB - 16 MiB, strides up to
+// 512 B past the row, and halo regions (one pack and one unpack, three sets of
+// buffers in turn), the former picks (the selector's, or for requests under
+// 1 MiB the rule's for single copies) -> this rule on MI355X:
+//                                              pack          unpack
+//   2 000, rows of 4 B - 4 KiB               2.39 -> 2.24   2.72 -> 1.94 ms
+//   the same, all multiples of 16 B apart    2.69 -> 2.36   2.41 -> 2.05 ms
+//   2 000, rows of 1 - 224 B, odd lengths    5.51 -> 5.02   8.15 -> 6.54 ms
+//   4 000 of up to 1 MiB, rows 1 - 224 B     1.27 -> 0.83   1.94 -> 0.89 ms
+//   64 subdomains of 128^3 doubles, radius 3      257 -> 235 us together
+// Each length's variant is the best or within 1 % of it over sixteen such
+// random batches.  Rows to or from host memory are bound by the link, which
+// the dword kernel keeps fullest (48 MiB of 4-KiB rows packed at 57.2 GB/s,
+// 53.1 with 16-B words; unpacked 55.5 and 54.4).  Small batches keep the
+// selector's picks: the three faces of a 512^3 grid took 9.26 us with them,
+// 9.91 us with the closed-form rule's.
+int saturated_variant(const Geom &g, int dir) {
+  const int64_t L = g.L;
+  const bool pack = dir == TEMPI_DIR_PACK;
+  if (g.host) {
+    return 9;
+  }
+  if (L >= 256) {
+    return pack && L > 512 ? 3 : 4;
+  }
+  if (L >= 128) {
+    return 5;
+  }
+  if (L >= 48) {
+    return 6;
+  }
+  if (L >= 24) {
+    return pack ? 17 : 7;
+  }
+  return L < 16 || L >= 20 ? 12 : 7;
+}
+
+bool saturated(const std::vector<Req> &rs) {
   uint64_t tiles = 0;
-  for (const Req &q : *rs) {
+  for (const Req &q : rs) {
     tiles += tiles_of(q);
   }
-  if (tiles <= (uint64_t)device_cu_count() * 8) {
-    return;
-  }
+  return tiles > (uint64_t)device_cu_count() * 8;
+}
+
+// gives the requests whose variant was left to the library `pick`'s
+template <class Pick>
+void repick(const tempi_batch_request *reqs, const std::vector<int64_t> &where,
+            std::vector<Req> *rs, Pick &&pick) {
   for (size_t k = 0; k < rs->size(); ++k) {
-    Req &q = (*rs)[k];
     const int asked = reqs[where[k]].variant;
-    if ((asked < 0 || asked >= kNumVariants) && q.g.L * q.g.rows < (1ll << 20)) {
-      q.variant = heuristic_variant(q.g, q.ds, q.dp, q.dir);
+    if (asked < 0 || asked >= kNumVariants) {
+      (*rs)[k].variant = pick((*rs)[k]);
     }
   }
+}
+
+// the variant that splits a request into the fewest tiles
+int fewest_tiles(const Req &q) {
+  Req r = q;
+  uint64_t best = UINT64_MAX;
+  int variant = q.variant;
+  for (r.variant = 0; r.variant < kNumVariants; ++r.variant) {
+    const uint64_t t = tiles_of(r);
+    if (t < best) {
+      best = t;
+      variant = r.variant;
+    }
+  }
+  return variant;
 }
 
 } // namespace
@@ -593,7 +648,7 @@ TEMPI_EXPORT int tempi_batch_create(const tempi_batch_request *reqs, int64_t n,
   // the per-copy policy first (in small batches the learned selector's
   // picks for requests under 1 MiB ran the faces of 128^3 - 256^3 float
   // grids 5-28 % faster than the closed-form rule's), then the batch rule
-  // for batches that saturate the grid (saturated_batch_policy).  The
+  // for batches that saturate the grid (saturated_variant).  The
   // selector evaluates all the batch's new shapes in one inference first:
   // one launch per shape took 0.14 s to create the 4 096-request batch.
   int err = resolve_requests(
@@ -618,9 +673,9 @@ TEMPI_EXPORT int tempi_batch_create(const tempi_batch_request *reqs, int64_t n,
                       .variant;
     }
   }
-  if (method == TEMPI_SELECT_DEFAULT) {
-    saturated_batch_policy(reqs, where, &rs);
-    //stream_batch(reqs, where, &rs);
+  if (method == TEMPI_SELECT_DEFAULT && saturated(rs)) {
+    repick(reqs, where, &rs,
+           [](const Req &q) { return saturated_variant(q.g, q.dir); });
   }
   for (size_t k = 0; k < rs.size(); ++k) {
     b->variants[(size_t)where[k]] = rs[k].variant;
@@ -931,10 +986,20 @@ TEMPI_EXPORT int tempi_batch_run_noalloc(const tempi_batch_request *reqs,
   if (rs.empty()) {
     return TEMPI_SUCCESS;
   }
-  //stream_batch(reqs, where, &rs);
+  if (saturated(rs)) {
+    repick(reqs, where, &rs,
+           [](const Req &q) { return saturated_variant(q.g, q.dir); });
+  }
   BatchPlan pl;
   if ((err = plan_batch(rs, &pl))) {
     return err;
+  }
+  if (pl.image.size() > kScratchBytes) {
+    // as many requests as the array can hold
+    repick(reqs, where, &rs, fewest_tiles);
+    if ((err = plan_batch(rs, &pl))) {
+      return err;
+    }
   }
   if (pl.image.size() > kScratchBytes) {
     return set_error(TEMPI_ERR_UNSUPPORTED,
