@@ -41,6 +41,17 @@ struct BatchItem {
 
 constexpr uint32_t kXcds = 8;
 
+// Units a lane of a tile keeps in flight.  In address order (`run`), among
+// tiles of other requests, two rows per lane are enough, and four fetch lines
+// before those of their neighbours are done with: 254 unpacks of 4-B rows
+// 4 - 516 B apart 799 us with two, 1 013 us with four, 238 of 8-B rows 421 and
+// 509 us.  A batch of few requests has the device to itself and takes all four:
+// the three faces of a 512^3 float grid, pack + unpack, 20.6 us with two,
+// 19.3 us with four.
+__host__ __device__ constexpr int units_per_lane(int P, int U, bool run) {
+  return run && P == 1 && units_in_flight(U) > 2 ? 2 : units_in_flight(U);
+}
+
 // One block-pass: tile `l` of a request split into `nt` tiles moves K blocks
 // of GROUPS units.  RUN: the K * GROUPS units from l * K * GROUPS on, so that
 // tiles in address order walk the memory in address order.  Else the blocks
@@ -54,8 +65,8 @@ template <int P, int W, int U, bool WHOLE, int DIR, bool NTS, bool NTL,
 __device__ __forceinline__ void copy_tile(const KParams &p, uint32_t l,
                                           uint32_t nt) {
   constexpr uint32_t GROUPS = kBlock / P;
-  constexpr uint32_t K = units_in_flight(U);
-  copy_units<P, W, U, WHOLE, DIR, NTS, NTL>(
+  constexpr uint32_t K = units_per_lane(P, U, RUN);
+  copy_units<P, W, U, WHOLE, DIR, NTS, NTL, K>(
       p, l * (RUN ? K * GROUPS : GROUPS) + threadIdx.x / P,
       RUN ? GROUPS : nt * GROUPS, p.units, threadIdx.x % P);
 }
@@ -214,6 +225,10 @@ struct BatchLaunch {
   const uint32_t *xcd_begin = nullptr; // first tile of each XCD (kXcds + 1)
 };
 
+uint32_t units_per_tile(const VariantDesc &v, bool run) {
+  return (uint32_t)(kBlock / v.P) * units_per_lane(v.P, v.U, run);
+}
+
 void launch_kernel(const BatchLaunch &l, hipStream_t s) {
   if (l.small) {
     hipLaunchKernelGGL(k_batch_small, dim3(l.grid), dim3(kBlock), 0, s, l.ix,
@@ -338,6 +353,7 @@ int plan_tables(const std::vector<Req> &rs, BatchPlan *pl) {
   std::vector<BatchItem> items;
   std::vector<uint32_t> item_tiles; // tiles of each item
   uint64_t tiles = 0;
+  const bool small = rs.size() <= (size_t)kSmallItems;
   for (const Req &r : rs) {
     BatchItem it{};
     bool whole = false;
@@ -347,7 +363,7 @@ int plan_tables(const std::vector<Req> &rs, BatchPlan *pl) {
     }
     it.kind = 4 * r.variant + 2 * (whole ? 1 : 0) + r.dir;
     const VariantDesc &v = kVariants[r.variant];
-    it.units_per_tile = (uint32_t)(kBlock / v.P) * units_in_flight(v.U);
+    it.units_per_tile = units_per_tile(v, !small);
     const uint64_t t = ((uint64_t)it.p.units + it.units_per_tile - 1) /
                        it.units_per_tile;
     tiles += t;
@@ -366,7 +382,7 @@ int plan_tables(const std::vector<Req> &rs, BatchPlan *pl) {
   // 3.81 ms.
   // (A launch has fewer than 2^32 threads: beyond 2^23 tiles the grid loops.)
   constexpr int64_t cap = 1 << 23;
-  if (!items.empty() && items.size() <= (size_t)kSmallItems) {
+  if (!items.empty() && small) {
     // tile index in the kernel arguments; only the parameters go to the
     // device table
     SmallIndex &ix = L.ix;
@@ -536,13 +552,14 @@ int build_batch(tempi_batch *b, const std::vector<Req> &rs) {
   return TEMPI_SUCCESS;
 }
 
-// Tiles of a resolved request (one workgroup pass each).
-uint64_t tiles_of(const Req &q) {
+// Tiles of a resolved request (one workgroup pass each); `run`: in a batch of
+// more than kSmallItems.
+uint64_t tiles_of(const Req &q, bool run) {
   const VariantDesc &v = kVariants[q.variant];
   const int64_t per_unit = (int64_t)v.P * v.U;
   const int64_t nseg = std::max<int64_t>(1, (q.g.L / v.W + per_unit - 1) / per_unit);
   const uint64_t units = (uint64_t)(q.g.rows * nseg);
-  const uint64_t per_tile = (uint64_t)(kBlock / v.P) * units_in_flight(v.U);
+  const uint64_t per_tile = units_per_tile(v, run);
   return (units + per_tile - 1) / per_tile;
 }
 
@@ -599,7 +616,7 @@ int saturated_variant(const Geom &g, int dir) {
 bool saturated(const std::vector<Req> &rs) {
   uint64_t tiles = 0;
   for (const Req &q : rs) {
-    tiles += tiles_of(q);
+    tiles += tiles_of(q, rs.size() > (size_t)kSmallItems);
   }
   return tiles > (uint64_t)device_cu_count() * 8;
 }
@@ -622,7 +639,7 @@ int fewest_tiles(const Req &q) {
   uint64_t best = UINT64_MAX;
   int variant = q.variant;
   for (r.variant = 0; r.variant < kNumVariants; ++r.variant) {
-    const uint64_t t = tiles_of(r);
+    const uint64_t t = tiles_of(r, true);
     if (t < best) {
       best = t;
       variant = r.variant;

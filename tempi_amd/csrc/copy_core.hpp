@@ -220,11 +220,11 @@ __host__ __device__ constexpr int units_in_flight(int U) {
 // in front of the later ones (register reuse across the grid-stride loop),
 // and each unit paid a full memory round trip of its own.  NTS / NTL:
 // nontemporal stores / loads of the body words.
-template <int P, int W, int U, bool WHOLE, int DIR, bool NTS, bool NTL>
+template <int P, int W, int U, bool WHOLE, int DIR, bool NTS, bool NTL,
+          int K = units_in_flight(U)>
 __device__ __forceinline__ void copy_units(const KParams &p, uint32_t first,
                                            uint32_t stride, uint32_t end,
                                            uint32_t lane) {
-  constexpr int K = units_in_flight(U);
   UnitAddr a[K];
 #pragma unroll
   for (int k = 0; k < K; ++k) {
@@ -311,11 +311,11 @@ enum Nontemporal { kPlain, kLoads, kStrided };
   X(9, 1, 4, 4, kPlain)     /* lane per row, 4-B words             */          \
   X(10, 16, 4, 4, kPlain)   /* 4-B words across 16 lanes           */          \
   X(11, 1, 1, 16, kPlain)   /* lane per row, bytes                 */          \
-  X(12, 1, 12, 2, kPlain)   /* lane per row, 12-B words (3 floats) */          \
+  X(12, 1, 12, 1, kPlain)   /* lane per row, 12-B words (3 floats) */          \
   X(13, 8, 16, 2, kLoads)   /* as 5, nontemporal loads             */          \
   X(14, 4, 16, 2, kStrided) /* as 6, strided side nontemporal      */          \
   X(15, 4, 16, 2, kLoads)   /* as 6, nontemporal loads             */          \
-  X(16, 1, 12, 2, kLoads)   /* as 12, nontemporal loads            */          \
+  X(16, 1, 12, 1, kLoads)   /* as 12, nontemporal loads            */          \
   X(17, 4, 8, 1, kLoads)    /* rows of 8 - 32 B, nontemporal loads */          \
   X(18, 1, 8, 4, kLoads)    /* as 8, nontemporal loads             */
 
