@@ -35,21 +35,24 @@ struct BatchItem {
   int32_t kind;            // 4 * variant + 2 * whole rows + direction
   uint32_t units_per_tile; // units of one block-pass: groups per block * K
   uint32_t ntiles;         // tiles of this request
-  uint32_t pad;
+  uint32_t two;            // two units per lane instead of four (two_or_four)
   KParams p;               // after the kind: both in the item's first lines
 };
 
 constexpr uint32_t kXcds = 8;
 
-// Units a lane of a tile keeps in flight.  In address order (`run`), among
-// tiles of other requests, two rows per lane are enough, and four fetch lines
-// before those of their neighbours are done with: 254 unpacks of 4-B rows
-// 4 - 516 B apart 799 us with two, 1 013 us with four, 238 of 8-B rows 421 and
-// 509 us.  A batch of few requests has the device to itself and takes all four:
-// the three faces of a 512^3 float grid, pack + unpack, 20.6 us with two,
-// 19.3 us with four.
-__host__ __device__ constexpr int units_per_lane(int P, int U, bool run) {
-  return run && P == 1 && units_in_flight(U) > 2 ? 2 : units_in_flight(U);
+// Lane-per-row variants of one-word units keep four units of a lane in flight,
+// or, where BatchItem::two is set, two.  Among tiles of other requests, in
+// address order, two are enough, and four fetch lines before those of their
+// neighbours are done with: 254 unpacks of 4-B rows 4 - 516 B apart took 799 us
+// with two, 1 013 us with four, 238 of 8-B rows 421 and 509 us.  A batch of few
+// requests has the device to itself and takes four: the three faces of a 512^3
+// float grid, pack + unpack, 20.6 us with two, 19.3 us with four.  Its requests
+// of less than 3/4 of a tile per CU take two again, for twice the workgroups
+// (320^3, 100 tiles of four: 11.6 us with four, 11.1 with two; 384^3, 144: 13.4
+// and 13.2; 448^3, 196: 16.1 and 16.4).
+__host__ __device__ constexpr bool two_or_four(int P, int U) {
+  return P == 1 && units_in_flight(U) > 2;
 }
 
 // One block-pass: tile `l` of a request split into `nt` tiles moves K blocks
@@ -63,21 +66,29 @@ __host__ __device__ constexpr int units_per_lane(int P, int U, bool run) {
 template <int P, int W, int U, bool WHOLE, int DIR, bool NTS, bool NTL,
           bool RUN>
 __device__ __forceinline__ void copy_tile(const KParams &p, uint32_t l,
-                                          uint32_t nt) {
+                                          uint32_t nt, bool two) {
   constexpr uint32_t GROUPS = kBlock / P;
-  constexpr uint32_t K = units_per_lane(P, U, RUN);
-  copy_units<P, W, U, WHOLE, DIR, NTS, NTL, K>(
+  if constexpr (two_or_four(P, U)) {
+    if (two) {
+      copy_units<P, W, U, WHOLE, DIR, NTS, NTL, 2>(
+          p, l * (RUN ? 2 * GROUPS : GROUPS) + threadIdx.x,
+          RUN ? GROUPS : nt * GROUPS, p.units, 0);
+      return;
+    }
+  }
+  constexpr uint32_t K = units_in_flight(U);
+  copy_units<P, W, U, WHOLE, DIR, NTS, NTL>(
       p, l * (RUN ? K * GROUPS : GROUPS) + threadIdx.x / P,
       RUN ? GROUPS : nt * GROUPS, p.units, threadIdx.x % P);
 }
 
 template <bool RUN>
 __device__ __forceinline__ void run_tile(int kind, const KParams &p,
-                                         uint32_t l, uint32_t nt) {
+                                         uint32_t l, uint32_t nt, bool two) {
   switch (kind) {
 #define TEMPI_BTILE(P, W, U, WHOLE, DIR, NT)                                   \
   copy_tile<P, W, U, WHOLE, DIR, nt_stores(NT, DIR), nt_loads(NT, DIR), RUN>(  \
-      p, l, nt);                                                               \
+      p, l, nt, two);                                                          \
   break;
 #define TEMPI_BCASE(I, P, W, U, NT)                                            \
   case 4 * I + 0:                                                              \
@@ -133,7 +144,7 @@ __global__ void __launch_bounds__(kBlock)
     const uint32_t r = __builtin_amdgcn_readfirstlane(tl.item);
     const uint32_t l = __builtin_amdgcn_readfirstlane(tl.tile);
     const BatchItem &it = items[r];
-    run_tile<true>(it.kind, it.p, l, it.ntiles);
+    run_tile<true>(it.kind, it.p, l, it.ntiles, it.two != 0);
   }
 }
 
@@ -198,7 +209,7 @@ __global__ void __launch_bounds__(kBlock)
     const uint32_t l = (q % kXcds) * sh + q / kXcds;
     if (l < nt) {
       const BatchItem &it = items[r];
-      run_tile<false>(it.kind, it.p, l, nt);
+      run_tile<false>(it.kind, it.p, l, nt, it.two != 0);
     }
   }
 }
@@ -225,8 +236,9 @@ struct BatchLaunch {
   const uint32_t *xcd_begin = nullptr; // first tile of each XCD (kXcds + 1)
 };
 
-uint32_t units_per_tile(const VariantDesc &v, bool run) {
-  return (uint32_t)(kBlock / v.P) * units_per_lane(v.P, v.U, run);
+uint32_t units_per_tile(const VariantDesc &v, bool two) {
+  return (uint32_t)(kBlock / v.P) *
+         (two && two_or_four(v.P, v.U) ? 2 : units_in_flight(v.U));
 }
 
 void launch_kernel(const BatchLaunch &l, hipStream_t s) {
@@ -246,6 +258,7 @@ struct Req {
   char *dp = nullptr;       // first packed byte (device address)
   int dir = 0;
   int variant = 0;
+  bool wide = false; // four units per lane where two would be taken
 };
 
 // The host image of a batch's device tables (request parameters, tile
@@ -363,7 +376,10 @@ int plan_tables(const std::vector<Req> &rs, BatchPlan *pl) {
     }
     it.kind = 4 * r.variant + 2 * (whole ? 1 : 0) + r.dir;
     const VariantDesc &v = kVariants[r.variant];
-    it.units_per_tile = units_per_tile(v, !small);
+    it.two = small ? (uint64_t)it.p.units * 4 <
+                         (uint64_t)units_per_tile(v, false) * device_cu_count() * 3
+                   : !r.wide;
+    it.units_per_tile = units_per_tile(v, it.two != 0);
     const uint64_t t = ((uint64_t)it.p.units + it.units_per_tile - 1) /
                        it.units_per_tile;
     tiles += t;
@@ -552,14 +568,14 @@ int build_batch(tempi_batch *b, const std::vector<Req> &rs) {
   return TEMPI_SUCCESS;
 }
 
-// Tiles of a resolved request (one workgroup pass each); `run`: in a batch of
-// more than kSmallItems.
-uint64_t tiles_of(const Req &q, bool run) {
+// Tiles of a resolved request (one workgroup pass each) in a batch of more
+// than kSmallItems.
+uint64_t tiles_of(const Req &q) {
   const VariantDesc &v = kVariants[q.variant];
   const int64_t per_unit = (int64_t)v.P * v.U;
   const int64_t nseg = std::max<int64_t>(1, (q.g.L / v.W + per_unit - 1) / per_unit);
   const uint64_t units = (uint64_t)(q.g.rows * nseg);
-  const uint64_t per_tile = units_per_tile(v, run);
+  const uint64_t per_tile = units_per_tile(v, !q.wide);
   return (units + per_tile - 1) / per_tile;
 }
 
@@ -616,7 +632,7 @@ int saturated_variant(const Geom &g, int dir) {
 bool saturated(const std::vector<Req> &rs) {
   uint64_t tiles = 0;
   for (const Req &q : rs) {
-    tiles += tiles_of(q, rs.size() > (size_t)kSmallItems);
+    tiles += tiles_of(q);
   }
   return tiles > (uint64_t)device_cu_count() * 8;
 }
@@ -639,7 +655,7 @@ int fewest_tiles(const Req &q) {
   uint64_t best = UINT64_MAX;
   int variant = q.variant;
   for (r.variant = 0; r.variant < kNumVariants; ++r.variant) {
-    const uint64_t t = tiles_of(r, true);
+    const uint64_t t = tiles_of(r);
     if (t < best) {
       best = t;
       variant = r.variant;
@@ -1012,7 +1028,10 @@ TEMPI_EXPORT int tempi_batch_run_noalloc(const tempi_batch_request *reqs,
     return err;
   }
   if (pl.image.size() > kScratchBytes) {
-    // as many requests as the array can hold
+    // as many rows to a tile record as a kernel moves
+    for (Req &q : rs) {
+      q.wide = true;
+    }
     repick(reqs, where, &rs, fewest_tiles);
     if ((err = plan_batch(rs, &pl))) {
       return err;

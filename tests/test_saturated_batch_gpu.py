@@ -81,7 +81,8 @@ def test_more_tiles_than_one_launch_starts(extra):
     out = torch.zeros(n, rows, dtype=torch.uint8, device="cuda")
     small = torch.zeros(8, 64, dtype=torch.uint8, device="cuda")
     torch.cuda.synchronize()
-    reqs = [(sb, src.data_ptr(), out[i].data_ptr(), 1, ta.DIR_PACK) for i in range(n)]
+    # the byte variant: 256 rows a tile
+    reqs = [(sb, src.data_ptr(), out[i].data_ptr(), 1, ta.DIR_PACK, 11) for i in range(n)]
     reqs += [(ta.StridedBlock.make(0, 0, [8, 8], [1, 16]), src.data_ptr(),
               small[i].data_ptr(), 1, ta.DIR_PACK) for i in range(extra)]
     b = ta.Batch(reqs)
@@ -93,3 +94,54 @@ def test_more_tiles_than_one_launch_starts(extra):
         assert torch.equal(out[i], want), i
     for i in range(extra):
         assert torch.equal(small[i], src[:128].view(8, 16)[:, :8].reshape(-1)), i
+
+
+@pytest.mark.parametrize("L", [12, 13])
+@pytest.mark.parametrize("variant", [12, 16])
+def test_few_requests_of_one_word_units(L, variant):
+    # two or four rows per lane, by the request's rows against 3/4 of a tile of
+    # 1 024 per CU (256 CUs: 196 608); and a request of less than one tile
+    rows = [196607, 196608, 196609, 600]
+    span = max(rows) * 24 + 64
+    host = orc.splitmix_bytes(span, 73)
+    src = ta.DeviceBuffer(span)
+    src.upload(host)
+    packed = [ta.DeviceBuffer(n * L + 16) for n in rows]
+    dsts = [ta.DeviceBuffer(span) for _ in rows]
+    blocks = [ta.StridedBlock.make(4, 0, [L, n], [1, 24]) for n in rows]
+    for b in packed:
+        b.fill(0x5A)
+    for b in dsts:
+        b.fill(0xAB)
+    ta.Batch([(sb, src.addr(), p.addr(), 1, ta.DIR_PACK, variant)
+              for sb, p in zip(blocks, packed)]).launch()
+    ta.Batch([(sb, d.addr(), p.addr(), 1, ta.DIR_UNPACK, variant)
+              for sb, d, p in zip(blocks, dsts, packed)]).launch()
+    ta.synchronize()
+    for sb, p, d, n in zip(blocks, packed, dsts, rows):
+        desc = orc.sb_desc(*sb.as_tuple())
+        want = np.full(n * L + 16, 0x5A, np.uint8)
+        want[:n * L] = orc.sb_pack(desc, host, 0, 1)
+        assert (p.download() == want).all(), n
+        ref = np.full(span, 0xAB, np.uint8)
+        orc.sb_unpack(desc, want[:n * L], ref, 0, 1)
+        assert (d.download() == ref).all(), n
+
+
+def test_noalloc_takes_fewer_tiles_before_it_refuses():
+    # 9 x 35 M rows of a byte: 615 000 tiles of the rule's 512 rows are past
+    # the 524 288 the array holds, those of 1 024 rows are not
+    rows, n = 35_000_000, 9
+    host = orc.splitmix_bytes(2 * rows, 79)
+    src, out = ta.DeviceBuffer(2 * rows), ta.DeviceBuffer(n * rows)
+    src.upload(host)
+    sb = ta.StridedBlock.make(1, 0, [1, rows], [1, 2])
+    reqs = [(sb, src.addr(), out.addr(i * rows), 1, ta.DIR_PACK) for i in range(n)]
+    ta.batch_run_noalloc(reqs)
+    ta.synchronize()
+    got = out.download().reshape(n, rows)
+    for i in range(n):
+        assert (got[i] == host[1::2]).all(), i
+    with pytest.raises(ta.TempiError) as e:
+        ta.batch_run_noalloc(reqs * 2)
+    assert e.value.code == ta.TEMPI_ERR_UNSUPPORTED
