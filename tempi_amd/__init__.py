@@ -513,7 +513,7 @@ def batch_run_noalloc(requests, stream_=None):
 
 
 class Batch:
-    """A fixed set of pack/unpack requests run by one persistent kernel.
+    """A fixed set of pack/unpack requests run by one kernel launch.
 
     requests: iterable of (StridedBlock, strided_addr, packed_addr, count,
     direction[, variant])."""

@@ -587,12 +587,12 @@ uint64_t tiles_of(const Req &q) {
 // words' kernel whatever their length: a row is one unit of one or two
 // accesses there and a lane has two rows in flight, where the other
 // lane-per-row kernels hold four words of one row, most of which a short row
-// does not have.  Packs of rows of 24-47 B take four lanes of 8 B to a row,
-// and those and packs of rows over 512 B read nontemporal: the lines of a
-// halo's long rows are read once, and leave the caches to those its short
-// rows share.  Unpacks gain or lose by nontemporal loads with the size of
-// the batch (64 subdomains of 96^3, rows of 8 B, 78 -> 57 us, of 12 B 92 ->
-// 111) and do without.  Random requests of 4 KiB - 16 MiB, strides up to
+// does not have.  Unpacks of rows of 24-47 B take four lanes of 8 B to a
+// row, and those and unpacks of rows over 512 B read the packed bytes, which
+// nobody reads again, nontemporal: the caches are left to the lines that short
+// rows write in part.  Packs gain or lose by nontemporal loads with the size
+// of the batch (64 subdomains of 96^3, rows of 8 B, pack + unpack 78 -> 57 us,
+// of 12 B 92 -> 111) and do without.  Random requests of 4 KiB - 16 MiB, strides up to
 // 512 B past the row, and halo regions (one pack and one unpack, three sets of
 // buffers in turn), the former picks (the selector's, or for requests under
 // 1 MiB the rule's for single copies) -> this rule on MI355X:
@@ -601,21 +601,21 @@ uint64_t tiles_of(const Req &q) {
 //   the same, all multiples of 16 B apart    2.69 -> 2.36   2.41 -> 2.05 ms
 //   2 000, rows of 1 - 224 B, odd lengths    5.51 -> 5.02   8.15 -> 6.54 ms
 //   4 000 of up to 1 MiB, rows 1 - 224 B     1.27 -> 0.83   1.94 -> 0.89 ms
-//   64 subdomains of 128^3 doubles, radius 3      257 -> 235 us together
+//   64 subdomains of 128^3 doubles, radius 3      257 -> 232 us together
 // Each length's variant is the best or within 1 % of it over sixteen such
 // random batches.  Rows to or from host memory are bound by the link, which
-// the dword kernel keeps fullest (48 MiB of 4-KiB rows packed at 57.2 GB/s,
-// 53.1 with 16-B words; unpacked 55.5 and 54.4).  Small batches keep the
+// the dword kernel keeps fullest (48 MiB of 4-KiB rows unpacked at 57.2 GB/s,
+// 53.1 with 16-B words; packed 55.5 and 54.4).  Small batches keep the
 // selector's picks: the three faces of a 512^3 grid took 9.26 us with them,
 // 9.91 us with the closed-form rule's.
 int saturated_variant(const Geom &g, int dir) {
   const int64_t L = g.L;
-  const bool pack = dir == TEMPI_DIR_PACK;
+  const bool unpack = dir == TEMPI_DIR_UNPACK;
   if (g.host) {
     return 9;
   }
   if (L >= 256) {
-    return pack && L > 512 ? 3 : 4;
+    return unpack && L > 512 ? 3 : 4;
   }
   if (L >= 128) {
     return 5;
@@ -624,7 +624,7 @@ int saturated_variant(const Geom &g, int dir) {
     return 6;
   }
   if (L >= 24) {
-    return pack ? 17 : 7;
+    return unpack ? 17 : 7;
   }
   return L < 16 || L >= 20 ? 12 : 7;
 }
