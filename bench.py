@@ -397,7 +397,7 @@ def main():
             "workload": "3D subarray faces of a 518^3 float32 grid (512^3 + 3-cell ghost ring): "
                         "pack + unpack of the x, y, z faces (512x512x3, 512x3x512, 3x512x512)",
             "packed_bytes_per_step": packed_per_step,
-            "path": "tempi_batch_launch: one persistent-queue launch packs the 3 faces, one "
+            "path": "tempi_batch_launch: one batch launch packs the 3 faces, one "
                     "unpacks them (library stream)",
         },
         "bit_exact": bit_exact,

@@ -175,8 +175,8 @@ int tempi_variant_info_get(int variant, tempi_variant_info *info);
 /* Variant the library would use for this copy.  Under the default policy a
    copy of at most 1 MiB (128 KiB in rows under 64 B) takes a closed-form
    choice: it is bound by its launch, not by the kernel.  So does one of
-   512 KiB or more whose packed side is host memory: the link bounds it.  A copy of 64 MiB or
-   more is settled on its first run: the model's three best variants and the
+   512 KiB or more whose packed side is host memory: the link bounds it.  A
+   copy of 64 MiB or more is settled on its first run: the model's three best variants and the
    closed-form rule's pick are each timed once, cold, writing a scratch image
    of the destination (never the caller's buffers), and the fastest is kept
    for the shape; before that run this returns the model's pick. */
@@ -267,17 +267,19 @@ int tempi_launch_latency_us(int reps, float *host_us, float *device_us);
    kernel per MPI_Pack and synchronizes (src/internal/packer_2d.cu:101-108).
    A batch is a fixed set of pack and/or unpack requests (for example the 26
    faces, edges and corners of a 3D halo), resolved once into a
-   device-resident descriptor table; one launch runs a persistent kernel that
-   drains all of them (a batch of at most 8 requests passes its tile index
-   in the kernel arguments instead of a device tile table).  tempi_batch_graph_launch replays the same launch from
-   a captured hipGraph; it is slower than tempi_batch_launch on ROCm 7.2,
+   device-resident descriptor table; one launch runs a workgroup per tile of
+   16 KiB or so of all of them, in the order of the strided side's addresses
+   (a batch of at most 8 requests passes its tile index in the kernel arguments
+   instead of a device tile table).  tempi_batch_graph_launch replays the same
+   launch from a captured hipGraph; it is slower than tempi_batch_launch on ROCm 7.2,
    whose hipGraphLaunch costs about 17 us of host time against about 2.7 us
    for a kernel launch, and is for callers whose own step is a graph.
    Requests in one batch must be independent (no
    request writes bytes another reads or writes).  Nothing is synchronized:
    wait on the stream.  `method` (TEMPI_SELECT_*) picks the variant of each
    request that leaves it to the library (variant -1), as for a single copy
-   of that request. */
+   of that request; under the default policy a batch of more than 8 tiles per
+   CU picks by row length, direction and where the packed bytes are. */
 typedef struct tempi_batch_request {
   tempi_strided_block sb; /* layout of one object                          */
   const void *strided;    /* strided buffer origin (pack: in, unpack: out)  */
@@ -315,7 +317,9 @@ int tempi_batch_destroy(tempi_batch *batch);
    process ends, not to memory it allocates; nothing is allocated on the
    device and nothing waits for the launch.  Requests with variant -1 take
    the closed-form rule (TEMPI_SELECT_HEURISTIC: the learned selector and
-   trial timings would allocate).  Batches whose tables exceed the array
+   trial timings would allocate), in a batch of more than 8 tiles per CU the
+   rule by row length that such batches take, and where the tables would not
+   fit, the variants with the fewest tiles.  Batches whose tables exceed the array
    (about 4 000 requests, or 2^19 tiles) fail with TEMPI_ERR_UNSUPPORTED
    before any device work.  Every call on a GPU overwrites that GPU's
    array: calls on one stream follow each other in stream order, but calls
