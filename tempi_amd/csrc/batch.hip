@@ -32,17 +32,17 @@ namespace tempi {
 namespace {
 
 struct BatchItem {
-  int32_t kind;            // 4 * variant + 2 * whole rows + direction
+  int32_t kind;            // 4 * variant + 2 * whole rows + direction + kFour
   uint32_t units_per_tile; // units of one block-pass: groups per block * K
   uint32_t ntiles;         // tiles of this request
-  uint32_t two;            // two units per lane instead of four (two_or_four)
+  uint32_t pad;
   KParams p;               // after the kind: both in the item's first lines
 };
 
 constexpr uint32_t kXcds = 8;
 
 // Lane-per-row variants of one-word units keep four units of a lane in flight,
-// or, where BatchItem::two is set, two.  Among tiles of other requests, in
+// (kFour), or two.  Among tiles of other requests, in
 // address order, two are enough, and four fetch lines before those of their
 // neighbours are done with: 254 unpacks of 4-B rows 4 - 516 B apart took 799 us
 // with two, 1 013 us with four, 238 of 8-B rows 421 and 509 us.  A batch of few
@@ -50,10 +50,16 @@ constexpr uint32_t kXcds = 8;
 // float grid, pack + unpack, 20.6 us with two, 19.3 us with four.  Its requests
 // of less than 3/4 of a tile per CU take two again, for twice the workgroups
 // (320^3, 100 tiles of four: 11.6 us with four, 11.1 with two; 384^3, 144: 13.4
-// and 13.2; 448^3, 196: 16.1 and 16.4).
+// and 13.2; 448^3, 196: 16.1 and 16.4), and so do its packs, whose loads of a
+// line each then queue behind each other (the 512^3 faces alone, pack 9.4 us
+// with four, 8.8 with two; unpack 7.7 and 8.3).
 __host__ __device__ constexpr bool two_or_four(int P, int U) {
   return P == 1 && units_in_flight(U) > 2;
 }
+
+// added to the kind of a request whose lanes take four units instead of two:
+// past the other kinds (equal cases would not compile)
+constexpr int kFour = 128;
 
 // One block-pass: tile `l` of a request split into `nt` tiles moves K blocks
 // of GROUPS units.  RUN: the K * GROUPS units from l * K * GROUPS on, so that
@@ -64,43 +70,39 @@ __host__ __device__ constexpr bool two_or_four(int P, int U) {
 // 12-B rows 2 KiB apart (262 144 rows), the same as the single-copy kernels'
 // grid-stride order.
 template <int P, int W, int U, bool WHOLE, int DIR, bool NTS, bool NTL,
-          bool RUN>
+          bool RUN, bool FOUR>
 __device__ __forceinline__ void copy_tile(const KParams &p, uint32_t l,
-                                          uint32_t nt, bool two) {
+                                          uint32_t nt) {
   constexpr uint32_t GROUPS = kBlock / P;
-  if constexpr (two_or_four(P, U)) {
-    if (two) {
-      copy_units<P, W, U, WHOLE, DIR, NTS, NTL, 2>(
-          p, l * (RUN ? 2 * GROUPS : GROUPS) + threadIdx.x,
-          RUN ? GROUPS : nt * GROUPS, p.units, 0);
-      return;
-    }
+  constexpr uint32_t K =
+      two_or_four(P, U) && !FOUR ? 2 : units_in_flight(U);
+  if constexpr (two_or_four(P, U) || !FOUR) {
+    copy_units<P, W, U, WHOLE, DIR, NTS, NTL, K>(
+        p, l * (RUN ? K * GROUPS : GROUPS) + threadIdx.x / P,
+        RUN ? GROUPS : nt * GROUPS, p.units, threadIdx.x % P);
   }
-  constexpr uint32_t K = units_in_flight(U);
-  copy_units<P, W, U, WHOLE, DIR, NTS, NTL>(
-      p, l * (RUN ? K * GROUPS : GROUPS) + threadIdx.x / P,
-      RUN ? GROUPS : nt * GROUPS, p.units, threadIdx.x % P);
 }
 
 template <bool RUN>
 __device__ __forceinline__ void run_tile(int kind, const KParams &p,
-                                         uint32_t l, uint32_t nt, bool two) {
+                                         uint32_t l, uint32_t nt) {
   switch (kind) {
-#define TEMPI_BTILE(P, W, U, WHOLE, DIR, NT)                                   \
-  copy_tile<P, W, U, WHOLE, DIR, nt_stores(NT, DIR), nt_loads(NT, DIR), RUN>(  \
-      p, l, nt, two);                                                          \
-  break;
+#define TEMPI_BTILE(K, P, W, U, WHOLE, DIR, NT, FOUR)                          \
+  case K:                                                                      \
+    copy_tile<P, W, U, WHOLE, DIR, nt_stores(NT, DIR), nt_loads(NT, DIR), RUN, \
+              FOUR>(p, l, nt);                                                 \
+    break;
+#define TEMPI_BKINDS(K, P, W, U, NT, FOUR)                                     \
+  TEMPI_BTILE(K + 0, P, W, U, false, 0, NT, FOUR)                              \
+  TEMPI_BTILE(K + 1, P, W, U, false, 1, NT, FOUR)                              \
+  TEMPI_BTILE(K + 2, P, W, U, true, 0, NT, FOUR)                               \
+  TEMPI_BTILE(K + 3, P, W, U, true, 1, NT, FOUR)
 #define TEMPI_BCASE(I, P, W, U, NT)                                            \
-  case 4 * I + 0:                                                              \
-    TEMPI_BTILE(P, W, U, false, 0, NT)                                         \
-  case 4 * I + 1:                                                              \
-    TEMPI_BTILE(P, W, U, false, 1, NT)                                         \
-  case 4 * I + 2:                                                              \
-    TEMPI_BTILE(P, W, U, true, 0, NT)                                          \
-  case 4 * I + 3:                                                              \
-    TEMPI_BTILE(P, W, U, true, 1, NT)
+  TEMPI_BKINDS(4 * I, P, W, U, NT, false)                                      \
+  TEMPI_BKINDS(4 * I + kFour, P, W, U, NT, true)
     TEMPI_VARIANTS(TEMPI_BCASE)
 #undef TEMPI_BCASE
+#undef TEMPI_BKINDS
 #undef TEMPI_BTILE
   default:
     break;
@@ -144,7 +146,7 @@ __global__ void __launch_bounds__(kBlock)
     const uint32_t r = __builtin_amdgcn_readfirstlane(tl.item);
     const uint32_t l = __builtin_amdgcn_readfirstlane(tl.tile);
     const BatchItem &it = items[r];
-    run_tile<true>(it.kind, it.p, l, it.ntiles, it.two != 0);
+    run_tile<true>(it.kind, it.p, l, it.ntiles);
   }
 }
 
@@ -209,7 +211,7 @@ __global__ void __launch_bounds__(kBlock)
     const uint32_t l = (q % kXcds) * sh + q / kXcds;
     if (l < nt) {
       const BatchItem &it = items[r];
-      run_tile<false>(it.kind, it.p, l, nt, it.two != 0);
+      run_tile<false>(it.kind, it.p, l, nt);
     }
   }
 }
@@ -236,9 +238,9 @@ struct BatchLaunch {
   const uint32_t *xcd_begin = nullptr; // first tile of each XCD (kXcds + 1)
 };
 
-uint32_t units_per_tile(const VariantDesc &v, bool two) {
+uint32_t units_per_tile(const VariantDesc &v, bool four) {
   return (uint32_t)(kBlock / v.P) *
-         (two && two_or_four(v.P, v.U) ? 2 : units_in_flight(v.U));
+         (!four && two_or_four(v.P, v.U) ? 2 : units_in_flight(v.U));
 }
 
 void launch_kernel(const BatchLaunch &l, hipStream_t s) {
@@ -376,10 +378,15 @@ int plan_tables(const std::vector<Req> &rs, BatchPlan *pl) {
     }
     it.kind = 4 * r.variant + 2 * (whole ? 1 : 0) + r.dir;
     const VariantDesc &v = kVariants[r.variant];
-    it.two = small ? (uint64_t)it.p.units * 4 <
-                         (uint64_t)units_per_tile(v, false) * device_cu_count() * 3
-                   : !r.wide;
-    it.units_per_tile = units_per_tile(v, it.two != 0);
+    const bool four = small ? r.dir == TEMPI_DIR_UNPACK &&
+                                  (uint64_t)it.p.units * 4 >=
+                                      (uint64_t)units_per_tile(v, true) *
+                                          device_cu_count() * 3
+                            : r.wide;
+    if (four && two_or_four(v.P, v.U)) {
+      it.kind += kFour;
+    }
+    it.units_per_tile = units_per_tile(v, four);
     const uint64_t t = ((uint64_t)it.p.units + it.units_per_tile - 1) /
                        it.units_per_tile;
     tiles += t;
@@ -575,7 +582,7 @@ uint64_t tiles_of(const Req &q) {
   const int64_t per_unit = (int64_t)v.P * v.U;
   const int64_t nseg = std::max<int64_t>(1, (q.g.L / v.W + per_unit - 1) / per_unit);
   const uint64_t units = (uint64_t)(q.g.rows * nseg);
-  const uint64_t per_tile = units_per_tile(v, !q.wide);
+  const uint64_t per_tile = units_per_tile(v, q.wide);
   return (units + per_tile - 1) / per_tile;
 }
 
@@ -605,9 +612,9 @@ uint64_t tiles_of(const Req &q) {
 // Each length's variant is the best or within 1 % of it over sixteen such
 // random batches.  Rows to or from host memory are bound by the link, which
 // the dword kernel keeps fullest (48 MiB of 4-KiB rows unpacked at 57.2 GB/s,
-// 53.1 with 16-B words; packed 55.5 and 54.4).  Small batches keep the
-// selector's picks: the three faces of a 512^3 grid took 9.26 us with them,
-// 9.91 us with the closed-form rule's.
+// 53.1 with 16-B words; packed 55.5 and 54.4).  Batches of few
+// requests or few tiles keep the selector's picks: the three faces of a 512^3
+// grid took 9.26 us with them, 9.91 us with the closed-form rule's.
 int saturated_variant(const Geom &g, int dir) {
   const int64_t L = g.L;
   const bool unpack = dir == TEMPI_DIR_UNPACK;
@@ -630,6 +637,9 @@ int saturated_variant(const Geom &g, int dir) {
 }
 
 bool saturated(const std::vector<Req> &rs) {
+  if (rs.size() <= (size_t)kSmallItems) {
+    return false;
+  }
   uint64_t tiles = 0;
   for (const Req &q : rs) {
     tiles += tiles_of(q);
