@@ -278,8 +278,9 @@ int tempi_launch_latency_us(int reps, float *host_us, float *device_us);
    request writes bytes another reads or writes).  Nothing is synchronized:
    wait on the stream.  `method` (TEMPI_SELECT_*) picks the variant of each
    request that leaves it to the library (variant -1), as for a single copy
-   of that request; under the default policy a batch of more than 8 tiles per
-   CU picks by row length, direction and where the packed bytes are. */
+   of that request; under the default policy a batch of more than 8 requests
+   and 8 tiles per CU picks by row length, direction and where the packed
+   bytes are. */
 typedef struct tempi_batch_request {
   tempi_strided_block sb; /* layout of one object                          */
   const void *strided;    /* strided buffer origin (pack: in, unpack: out)  */
@@ -317,9 +318,9 @@ int tempi_batch_destroy(tempi_batch *batch);
    process ends, not to memory it allocates; nothing is allocated on the
    device and nothing waits for the launch.  Requests with variant -1 take
    the closed-form rule (TEMPI_SELECT_HEURISTIC: the learned selector and
-   trial timings would allocate), in a batch of more than 8 tiles per CU the
-   rule by row length that such batches take, and where the tables would not
-   fit, the variants with the fewest tiles.  Batches whose tables exceed the array
+   trial timings would allocate), in a batch of more than 8 requests and 8
+   tiles per CU the rule by row length that such batches take, and where the
+   tables would not fit, the variants with the fewest tiles.  Batches whose tables exceed the array
    (about 4 000 requests, or 2^19 tiles) fail with TEMPI_ERR_UNSUPPORTED
    before any device work.  Every call on a GPU overwrites that GPU's
    array: calls on one stream follow each other in stream order, but calls

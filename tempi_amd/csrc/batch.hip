@@ -41,18 +41,16 @@ struct BatchItem {
 
 constexpr uint32_t kXcds = 8;
 
-// Lane-per-row variants of one-word units keep four units of a lane in flight,
-// (kFour), or two.  Among tiles of other requests, in
-// address order, two are enough, and four fetch lines before those of their
-// neighbours are done with: 254 unpacks of 4-B rows 4 - 516 B apart took 799 us
-// with two, 1 013 us with four, 238 of 8-B rows 421 and 509 us.  A batch of few
-// requests has the device to itself and takes four: the three faces of a 512^3
-// float grid, pack + unpack, 20.6 us with two, 19.3 us with four.  Its requests
-// of less than 3/4 of a tile per CU take two again, for twice the workgroups
-// (320^3, 100 tiles of four: 11.6 us with four, 11.1 with two; 384^3, 144: 13.4
-// and 13.2; 448^3, 196: 16.1 and 16.4), and so do its packs, whose loads of a
-// line each then queue behind each other (the 512^3 faces alone, pack 9.4 us
-// with four, 8.8 with two; unpack 7.7 and 8.3).
+// Lane-per-row variants of one-word units keep four units of a lane in flight
+// (kFour) or two.  Among tiles of other requests, in address order, two are
+// enough, and four fetch lines before those of their neighbours are done with:
+// 254 unpacks of 4-B rows 4 - 516 B apart took 799 us with two, 1 013 us with
+// four, 238 of 8-B rows 421 and 509 us.  A batch of few requests has the device
+// to itself, and its unpacks take four: the three faces of a 512^3 float grid,
+// unpack alone, 8.3 us with two, 7.7 with four.  Its packs, whose loads of a
+// line each then queue behind each other, take two (8.8 us; 9.4 with four), and
+// so do requests of less than 3/4 of a tile per CU, for twice the workgroups
+// (pack + unpack, 320^3, 100 tiles of four: 11.1 us; 11.6 with four).
 __host__ __device__ constexpr bool two_or_four(int P, int U) {
   return P == 1 && units_in_flight(U) > 2;
 }
@@ -599,10 +597,10 @@ uint64_t tiles_of(const Req &q) {
 // nobody reads again, nontemporal: the caches are left to the lines that short
 // rows write in part.  Packs gain or lose by nontemporal loads with the size
 // of the batch (64 subdomains of 96^3, rows of 8 B, pack + unpack 78 -> 57 us,
-// of 12 B 92 -> 111) and do without.  Random requests of 4 KiB - 16 MiB, strides up to
-// 512 B past the row, and halo regions (one pack and one unpack, three sets of
-// buffers in turn), the former picks (the selector's, or for requests under
-// 1 MiB the rule's for single copies) -> this rule on MI355X:
+// of 12 B 92 -> 111) and do without.  Random requests of 4 KiB - 16 MiB, strides
+// up to 512 B past the row, and halo regions (one pack and one unpack, three
+// sets of buffers in turn), the former picks (the selector's, or for requests
+// under 1 MiB the rule's for single copies) -> this rule on MI355X:
 //                                              pack          unpack
 //   2 000, rows of 4 B - 4 KiB               2.39 -> 2.24   2.72 -> 1.94 ms
 //   the same, all multiples of 16 B apart    2.69 -> 2.36   2.41 -> 2.05 ms
@@ -612,9 +610,9 @@ uint64_t tiles_of(const Req &q) {
 // Each length's variant is the best or within 1 % of it over sixteen such
 // random batches.  Rows to or from host memory are bound by the link, which
 // the dword kernel keeps fullest (48 MiB of 4-KiB rows unpacked at 57.2 GB/s,
-// 53.1 with 16-B words; packed 55.5 and 54.4).  Batches of few
-// requests or few tiles keep the selector's picks: the three faces of a 512^3
-// grid took 9.26 us with them, 9.91 us with the closed-form rule's.
+// 53.1 with 16-B words; packed 55.5 and 54.4).  Batches of few requests or few
+// tiles keep the selector's picks: the three faces of a 512^3 grid took 9.26 us
+// with them, 9.91 us with the closed-form rule's.
 int saturated_variant(const Geom &g, int dir) {
   const int64_t L = g.L;
   const bool unpack = dir == TEMPI_DIR_UNPACK;
