@@ -268,8 +268,8 @@ int streamed_variant(int variant, const Geom &g, const char *strided, int dir,
 // the variant for a copy that runs alone and is bound by its launch; -1: it
 // is too large for that
 int latency_variant(const Geom &g);
-// the variant for a copy that runs alone and whose packed side is host
-// memory; -1: it is too small to be bound by the link
+// the variant for a copy whose packed side is host memory; -1: it is too small
+// to be bound by the link
 int link_variant(const Geom &g, int dir);
 
 // a kernel variant and its grid cap (0: the default cap)

@@ -146,3 +146,29 @@ def test_noalloc_takes_fewer_tiles_before_it_refuses():
     with pytest.raises(ta.TempiError) as e:
         ta.batch_run_noalloc(reqs * 2)
     assert e.value.code == ta.TEMPI_ERR_UNSUPPORTED
+
+
+def test_few_requests_from_host_memory():
+    # unpacks of 512 KiB and more read mapped memory lane apart, in dwords
+    sizes = [(12, 50000, 100), (1024, 700, 1100), (100, 100, 130)]  # the last is small
+    blocks = [ta.StridedBlock.make(5, 0, [L, n], [1, st]) for L, n, st in sizes]
+    span = max(n * st for _, n, st in sizes) + 64
+    packed = ta.DeviceBuffer(sum(sb.size() for sb in blocks) + 3, mapped=True)
+    host = orc.splitmix_bytes(packed.nbytes, 83)
+    packed.upload(host)
+    dsts = [ta.DeviceBuffer(span) for _ in blocks]
+    reqs, at = [], 0
+    for sb, d in zip(blocks, dsts):
+        d.fill(0xAB)
+        reqs.append((sb, d.addr(), packed.addr(at), 1, ta.DIR_UNPACK))
+        at += sb.size() + 1  # odd packed addresses
+    b = ta.Batch(reqs)
+    assert [b.variant(i) for i in range(2)] == [9, 9]
+    b.launch()
+    ta.synchronize()
+    at = 0
+    for sb, d in zip(blocks, dsts):
+        ref = np.full(span, 0xAB, np.uint8)
+        orc.sb_unpack(orc.sb_desc(*sb.as_tuple()), host[at:at + sb.size()], ref, 0, 1)
+        assert (d.download() == ref).all()
+        at += sb.size() + 1
