@@ -420,6 +420,10 @@ typedef struct tempi_counters {
 } tempi_counters;
 int tempi_counters_get(tempi_counters *out);
 int tempi_counters_reset(void);
+/* Completion signals of this process so far: `numbers`, the last number given
+   to one (each is given once), and `kernels`, those sent by a kernel behind
+   their copy rather than by the copy's last workgroup. */
+int tempi_signals_get(int64_t *numbers, int64_t *kernels);
 
 /* ---- measured system performance and the send-method model ----------------
    The reference's system model (include/measure_system.hpp:26-106,

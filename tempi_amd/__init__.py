@@ -208,6 +208,7 @@ def _prototypes(L):
                                 ctypes.POINTER(ctypes.c_float)]),
         "tempi_copy_emulate": (_I, [sb_p, _I64, ctypes.c_uint64, ctypes.c_uint64, _I, _I, _I, _I,
                                     _I64, ctypes.POINTER(CopyEmulation)]),
+        "tempi_signals_get": (_I, [i64_p, i64_p]),
         "tempi_flush_caches": (_I, [_I64]),
         "tempi_launch_latency_us": (_I, [_I, ctypes.POINTER(ctypes.c_float),
                                          ctypes.POINTER(ctypes.c_float)]),
@@ -302,6 +303,14 @@ def counters() -> dict:
     c = Counters()
     check(lib().tempi_counters_get(ctypes.byref(c)))
     return c.as_dict()
+
+
+def signals() -> tuple:
+    """(last number given to a completion signal, signals sent by a kernel
+    behind their copy)."""
+    n, k = ctypes.c_int64(), ctypes.c_int64()
+    check(lib().tempi_signals_get(ctypes.byref(n), ctypes.byref(k)))
+    return n.value, k.value
 
 
 def reset_counters():

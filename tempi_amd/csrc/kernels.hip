@@ -616,7 +616,8 @@ struct SignalState {
   bool tried = false;
   SignalSlots slots{};       // device addresses: device memory, the flag
   uint32_t *flag = nullptr;  // pinned host memory
-  unsigned long long issued = 0; // signals so far
+  unsigned long long issued = 0; // the last number given to a signal
+  int64_t kernels = 0;           // signals sent by a kernel behind their work
   // set after a signalled wait fails: the counter may no longer match the
   // launches, so later copies wait on the stream
   std::atomic<bool> off{false};
@@ -627,11 +628,16 @@ SignalState &signal_state() {
   return s;
 }
 
-// The kernels store the low 32 bits of a signal's number; the next number
-// skips those that would read as none (the state's lock held).
-unsigned long long next_signal(const SignalState &st) {
-  const unsigned long long n = st.issued + 1;
-  return (uint32_t)n ? n : n + 1;
+// The next signal's number, given for good (the state's lock held).  A number
+// that may have reached the device is never given again: were it, the second
+// copy's wait would end on the first one's signal.  One whose launch failed is
+// skipped, as waits compare with >=, and so are those whose low 32 bits, which
+// the kernels store, would read as none.
+unsigned long long take_number(SignalState &st) {
+  do {
+    ++st.issued;
+  } while (!(uint32_t)st.issued);
+  return st.issued;
 }
 
 bool flag_at(const SignalState &st, unsigned long long seq) {
@@ -742,13 +748,21 @@ unsigned long long signal_stream() {
   if (!signal_ready(st)) {
     return 0;
   }
-  const unsigned long long n = next_signal(st);
-  hipLaunchKernelGGL(k_signal, dim3(1), dim3(1), 0, library_stream(),
-                     st.slots.flag, (uint32_t)n);
-  if (hipSuccess != hipGetLastError()) {
+  const unsigned long long n = take_number(st);
+  // judged by the launch's own result: hipGetLastError reports, and clears,
+  // whatever earlier error of this thread the application has not read yet
+  uint32_t number = (uint32_t)n;
+  void *args[] = {&st.slots.flag, &number};
+  const hipError_t e =
+      hipLaunchKernel(reinterpret_cast<const void *>(k_signal), dim3(1),
+                      dim3(1), args, 0, library_stream());
+  if (e != hipSuccess) {
+    (void)hipGetLastError(); // this launch's own
+    TEMPI_LOG(LOG_WARN, "signal kernel: %s", hipGetErrorString(e));
     return 0;
   }
-  return st.issued = n;
+  ++st.kernels;
+  return n;
 }
 
 int launch_copy_signalled(const Geom &g, const char *strided, char *packed,
@@ -767,11 +781,11 @@ int launch_copy_signalled(const Geom &g, const char *strided, char *packed,
     SignalState &st = signal_state();
     std::lock_guard<std::mutex> lk(st.mu);
     if (signal_ready(st)) {
-      const unsigned long long n = next_signal(st);
+      const unsigned long long n = take_number(st);
       const int err = launch_one(g, strided, packed, dir, variant, s,
                                  max_blocks, (uint32_t)n, st.slots);
       if (!err) {
-        *seq = st.issued = n;
+        *seq = n;
         *own = true;
       }
       return err;
@@ -930,6 +944,18 @@ const EmulateFn kEmulate[][2][2] = {TEMPI_VARIANTS(TEMPI_EROW)};
 } // namespace tempi
 
 using namespace tempi;
+
+TEMPI_EXPORT int tempi_signals_get(int64_t *numbers, int64_t *kernels) {
+  SignalState &st = signal_state();
+  std::lock_guard<std::mutex> lk(st.mu);
+  if (numbers) {
+    *numbers = (int64_t)st.issued;
+  }
+  if (kernels) {
+    *kernels = st.kernels;
+  }
+  return TEMPI_SUCCESS;
+}
 
 // Emulates launch_copy of the copy on the host (see above); `unit_limit`
 // bounds the work units emulated in full (beyond it only the launch plan is
