@@ -329,6 +329,26 @@ int tempi_batch_destroy(tempi_batch *batch);
 int tempi_batch_run_noalloc(const tempi_batch_request *reqs, int64_t n,
                             void *stream);
 
+/* Host-side plan of a batch: what tempi_batch_run_noalloc would launch for
+   these requests, without a device.  The requests' addresses are numbers
+   only; `packed_on_host` says that the packed ones are host memory.
+   `variants` (n entries, may be null) gets each request's variant, -1 where
+   it moves nothing.  Fails as tempi_batch_run_noalloc does, except that
+   tables over the static array are reported in fits_static_tables. */
+typedef struct tempi_batch_emulation {
+  int64_t requests;      /* requests that move something                    */
+  int64_t tiles;         /* workgroup passes                                */
+  int64_t grid;          /* workgroups of the launch                        */
+  int64_t xcd_tiles[8];  /* tiles that run on each XCD                      */
+  double xcd_bytes[8];   /* bytes of lines they move                        */
+  int32_t exact;         /* 1: every tile of every request runs once        */
+  int32_t fits_static_tables;
+} tempi_batch_emulation;
+int tempi_batch_emulate(const tempi_batch_request *reqs, int64_t n,
+                        int packed_on_host, int32_t *variants,
+                        tempi_batch_emulation *out);
+
+
 /* Learned variant selector: replaces the reference's measured tables and
    interpolation (src/internal/measure_system.cpp:181-299) and its fixed
    kernel rule (include/pack_kernels.cuh:129-166).  An MLP

@@ -144,6 +144,20 @@ class CopyEmulation(ctypes.Structure):
         return {n: getattr(self, n) for n, _ in self._fields_ if n != "reserved"}
 
 
+class BatchEmulation(ctypes.Structure):
+    """tempi_batch_emulation (include/tempi_amd.h)."""
+
+    _fields_ = [
+        ("requests", ctypes.c_int64),
+        ("tiles", ctypes.c_int64),
+        ("grid", ctypes.c_int64),
+        ("xcd_tiles", ctypes.c_int64 * 8),
+        ("xcd_bytes", ctypes.c_double * 8),
+        ("exact", ctypes.c_int32),
+        ("fits_static_tables", ctypes.c_int32),
+    ]
+
+
 class BatchRequest(ctypes.Structure):
     """tempi_batch_request (include/tempi_amd.h)."""
 
@@ -219,6 +233,9 @@ def _prototypes(L):
         "tempi_batch_variant": (_I, [_P, _I64, ctypes.POINTER(_I)]),
         "tempi_batch_destroy": (_I, [_P]),
         "tempi_batch_run_noalloc": (_I, [ctypes.POINTER(BatchRequest), _I64, _P]),
+        "tempi_batch_emulate": (_I, [ctypes.POINTER(BatchRequest), _I64, _I,
+                                     ctypes.POINTER(ctypes.c_int32),
+                                     ctypes.POINTER(BatchEmulation)]),
         "tempi_graph_create": (_I, [ctypes.POINTER(_P), _I64, ctypes.POINTER(_P)]),
         "tempi_graph_launch": (_I, [_P, _P]),
         "tempi_graph_destroy": (_I, [_P]),
@@ -519,6 +536,19 @@ def batch_run_noalloc(requests, stream_=None):
     asynchronous on the stream."""
     arr, n = batch_requests(requests)
     check(lib().tempi_batch_run_noalloc(arr, n, stream_), "batch_run_noalloc")
+
+
+def batch_emulate(requests, packed_on_host: bool = False) -> dict:
+    """The plan tempi_batch_run_noalloc would launch, from addresses that are
+    numbers only (no GPU); see tempi_batch_emulate."""
+    arr, n = batch_requests(requests)
+    variants = (ctypes.c_int32 * max(n, 1))()
+    out = BatchEmulation()
+    check(lib().tempi_batch_emulate(arr, n, int(packed_on_host), variants, ctypes.byref(out)),
+          "batch_emulate")
+    r = {name: getattr(out, name) for name, _ in out._fields_}
+    return dict(r, xcd_tiles=list(out.xcd_tiles), xcd_bytes=list(out.xcd_bytes),
+                variants=list(variants[:n]))
 
 
 class Batch:

@@ -272,91 +272,128 @@ struct BatchPlan {
 };
 
 // The tile records of a batch in the order of the strided side's addresses,
-// to windows of kWindowBytes, cut into `groups` consecutive ranges of about
-// equal traffic (begin[x] is the first tile of range x).  Requests of a batch
-// share lines -- a halo's faces, edges and corners, the low x face of a row
-// and the high one of the row before -- and partly written lines: with every
-// request in turn, and an eighth of each on every XCD, those lines were
-// fetched by several XCDs, or again after the L2 had dropped them; now one
-// XCD meets them at about the same time.  MI355X, request order -> address
-// order:
+// to windows of 4 KiB, cut into `groups` consecutive ranges of about
+// equal traffic (begin[x] is the first tile of range x; a range may end inside
+// a window).  Requests of a batch share lines -- a halo's faces, edges and
+// corners, the low x face of a row and the high one of the row before -- and
+// partly written lines: with every request in turn, and an eighth of each on
+// every XCD, those lines were fetched by several XCDs, or again after the L2
+// had dropped them; now one XCD meets them at about the same time.  MI355X,
+// request order -> address order:
 //   halo pack + unpack, 64 subdomains of 128^3 doubles   312 -> 276 us
 //   36 subdomains of 26^3 floats, radius 1               20.9 -> 7.7 us
 //   4 096 random requests from one source of 1.6 GB      5.59 -> 4.33 ms
 // (the last with windows of 64 KiB 4.39, of 256 KiB 4.96 ms).
 constexpr int kWindowShift = 12; // 4 KiB, wider where they would outnumber the tiles
 
-void order_tiles(const std::vector<Req> &rs, const std::vector<BatchItem> &items,
-                 uint64_t tiles, int groups, Tile *out, uint32_t *begin) {
-  // A request's tile l is taken to start at a + l * step: exact for rows at
-  // one stride, near enough for several dimensions.  Only the order depends
-  // on it.
-  struct Walk {
-    int64_t at;     // first tile's strided address, 12 fraction bits
-    int64_t step;   // from tile to tile, 12 fraction bits
-    float cost;     // bytes of lines a tile moves
+// [first, last) of the strided addresses a request touches
+void strided_range(const Req &q, uintptr_t *first, uintptr_t *last) {
+  const uintptr_t a = (uintptr_t)(q.ds + q.g.start);
+  *first = a;
+  *last = a + (uintptr_t)q.g.L;
+  for (int k = 0; k < q.g.nrd; ++k) {
+    const int64_t reach = (q.g.cnt[k] - 1) * q.g.str[k];
+    (reach < 0 ? *first : *last) += (uintptr_t)reach;
+  }
+}
+
+// What the tile order needs of each request.  A request's tile l is taken to
+// start at `at` + l * `step`: exact for rows at one stride, near enough for
+// several dimensions.  Only the order depends on it.
+struct Walk {
+  int64_t at;   // first tile's position, 12 fraction bits
+  int64_t step; // from tile to tile, 12 fraction bits
+  float cost;   // bytes of lines a tile moves
+};
+
+// The positions are the strided addresses with the memory between the
+// requests left out: two grids far apart would otherwise share the windows
+// with the gap between them and come out as one window each.  52 packs of 1 280
+// rows of 512 B from two grids of 20 MB, us, by the distance of the grids
+// (with the gap, ranges ending at windows -> without it, ending anywhere):
+//   20 MB 11.8 -> 11.8    16 GiB 16.1 -> 11.8    100 GiB 31.6 -> 11.7
+// and 1 000 packs of one 64-KiB region 17.2 -> 11.7.  Returns the length of the
+// occupied part.
+int64_t lay_out(const std::vector<Req> &rs, const std::vector<BatchItem> &items,
+                std::vector<Walk> *walk) {
+  struct Range {
+    uintptr_t first, last;
+    size_t r;
   };
   const size_t n = items.size();
-  std::vector<Walk> walk(n);
-  uintptr_t lo = UINTPTR_MAX, hi = 0;
+  std::vector<Range> ranges(n);
   for (size_t r = 0; r < n; ++r) {
-    const BatchItem &it = items[r];
-    const Geom &g = rs[r].g;
-    const uintptr_t a = (uintptr_t)(rs[r].ds + g.start);
+    strided_range(rs[r], &ranges[r].first, &ranges[r].last);
+    ranges[r].r = r;
+  }
+  std::sort(ranges.begin(), ranges.end(),
+            [](const Range &a, const Range &b) { return a.first < b.first; });
+  constexpr uintptr_t kWindow = (uintptr_t)1 << kWindowShift;
+  uintptr_t left_out = ranges[0].first / kWindow * kWindow;
+  uintptr_t end = ranges[0].first;
+  for (const Range &q : ranges) {
+    if (q.first > end) {
+      left_out += (q.first - end) / kWindow * kWindow;
+    }
+    end = std::max(end, q.last);
+    const BatchItem &it = items[q.r];
+    const Geom &g = rs[q.r].g;
+    Walk &w = (*walk)[q.r];
     const uint32_t last = it.ntiles - 1;
     const int64_t reach =
         last ? row_offset(it.p, it.p.segdiv.div(last * it.units_per_tile)) : 0;
-    walk[r].step = last ? reach * 4096 / (int64_t)last : 0;
+    w.at = (int64_t)((uintptr_t)(rs[q.r].ds + g.start) - left_out) * 4096;
+    w.step = last ? reach * 4096 / (int64_t)last : 0;
     if (g.rows == 1) {
-      walk[r].step = (int64_t)((double)g.L * 4096 / it.ntiles);
+      w.step = (int64_t)((double)g.L * 4096 / it.ntiles);
     }
-    walk[r].cost = (float)(((double)touched_bytes(g) + (double)g.L * g.rows) /
-                           it.ntiles);
-    lo = std::min(lo, reach < 0 ? a + (uintptr_t)reach : a);
-    hi = std::max(hi, reach < 0 ? a : a + (uintptr_t)std::max(reach, g.L));
+    w.cost = (float)(((double)touched_bytes(g) + (double)g.L * g.rows) / it.ntiles);
   }
+  return (int64_t)(end - left_out);
+}
+
+void order_tiles(const std::vector<Req> &rs, const std::vector<BatchItem> &items,
+                 uint64_t tiles, int groups, Tile *out, uint32_t *begin) {
+  const size_t n = items.size();
+  std::vector<Walk> walk(n);
+  const int64_t span = lay_out(rs, items, &walk);
   int shift = kWindowShift;
-  while (((hi - lo) >> shift) > 2 * tiles + 1024) {
+  while ((uint64_t)(span >> shift) > 2 * tiles + 1024) {
     ++shift;
   }
-  const int64_t windows = (int64_t)((hi - lo) >> shift) + 1;
+  const int64_t windows = (span >> shift) + 1;
   std::vector<uint32_t> at((size_t)windows + 1, 0);
-  std::vector<float> cost((size_t)windows, 0.0f);
-  double total = 0;
-  for (size_t r = 0; r < n; ++r) {
-    walk[r].at =
-        (int64_t)((uintptr_t)(rs[r].ds + rs[r].g.start) - lo) * 4096;
-    total += (double)walk[r].cost * items[r].ntiles;
-  }
   const auto window = [&](int64_t pos) {
     return std::min(std::max<int64_t>(pos >> (shift + 12), 0), windows - 1);
   };
+  double total = 0;
   for (size_t r = 0; r < n; ++r) {
     int64_t pos = walk[r].at;
     for (uint32_t l = 0; l < items[r].ntiles; ++l, pos += walk[r].step) {
-      const int64_t w = window(pos);
-      ++at[(size_t)w + 1];
-      cost[(size_t)w] += walk[r].cost;
+      ++at[(size_t)window(pos) + 1];
     }
+    total += (double)walk[r].cost * items[r].ntiles;
   }
-  double done = 0;
-  int x = 0;
-  begin[0] = 0;
   for (int64_t w = 0; w < windows; ++w) {
-    while (x + 1 < groups && done >= total * (x + 1) / groups) {
-      begin[++x] = at[(size_t)w];
-    }
-    done += cost[(size_t)w];
     at[(size_t)w + 1] += at[(size_t)w];
-  }
-  while (x + 1 < groups) {
-    begin[++x] = (uint32_t)tiles;
   }
   for (size_t r = 0; r < n; ++r) {
     int64_t pos = walk[r].at;
     for (uint32_t l = 0; l < items[r].ntiles; ++l, pos += walk[r].step) {
       out[at[(size_t)window(pos)]++] = Tile{(uint32_t)r, l};
     }
+  }
+  double done = 0;
+  int x = 0;
+  begin[0] = 0;
+  for (uint64_t t = 0; t < tiles && x + 1 < groups; ++t) {
+    done += walk[out[t].item].cost;
+    while (x + 1 < groups && done >= total * (x + 1) / groups) {
+      begin[++x] = (uint32_t)(t + 1);
+    }
+  }
+  while (x + 1 < groups) {
+    begin[++x] = (uint32_t)tiles;
   }
 }
 
@@ -472,10 +509,28 @@ BatchLaunch placed(const BatchPlan &pl, char *dev) {
 // for a request that leaves it to the library (variant -1), the variant
 // `pick` returns.  Requests that move nothing are left out; `where` gets
 // the caller's index of each resolved request.
-template <class Pick>
-int resolve_requests(const tempi_batch_request *reqs, int64_t n, Pick &&pick,
-                     std::vector<Req> *rs, std::vector<int64_t> *where,
-                     int64_t *bytes) {
+struct Resolved {
+  std::vector<Req> rs;
+  std::vector<int64_t> where;
+  int64_t bytes = 0;
+};
+
+// the addresses the kernels use for a request's buffers
+bool device_buffers(const tempi_batch_request &r, Req *q) {
+  void *ds = nullptr, *dp = nullptr;
+  if (!device_address(r.strided, &ds) ||
+      !device_address(r.packed, &dp, &q->g.host)) {
+    return false;
+  }
+  q->ds = static_cast<const char *>(ds);
+  q->dp = static_cast<char *>(dp);
+  return true;
+}
+
+template <class Buffers, class Pick>
+int resolve_requests(const tempi_batch_request *reqs, int64_t n,
+                     bool on_device, Buffers &&buffers, Pick &&pick,
+                     Resolved *out) {
   // every request is checked before the device is touched
   int err = TEMPI_SUCCESS;
   std::vector<Geom> geoms((size_t)n);
@@ -485,10 +540,9 @@ int resolve_requests(const tempi_batch_request *reqs, int64_t n, Pick &&pick,
       return err;
     }
   }
-  if ((err = ensure_runtime())) {
+  if (on_device && (err = ensure_runtime())) {
     return err;
   }
-  *bytes = 0;
   for (int64_t i = 0; i < n; ++i) {
     const tempi_batch_request &r = reqs[i];
     Req q;
@@ -501,22 +555,19 @@ int resolve_requests(const tempi_batch_request *reqs, int64_t n, Pick &&pick,
                        "request %lld: rows over 1 GiB are not batched",
                        (long long)i);
     }
-    void *ds = nullptr, *dp = nullptr;
-    if (!device_address(r.strided, &ds) || !device_address(r.packed, &dp, &q.g.host)) {
+    if (!buffers(r, &q)) {
       return set_error(TEMPI_ERR_ARG,
                        "request %lld: buffers must be device-accessible",
                        (long long)i);
     }
-    q.ds = static_cast<const char *>(ds);
-    q.dp = static_cast<char *>(dp);
     q.dir = r.direction;
     q.variant = r.variant;
     if (q.variant < 0 || q.variant >= kNumVariants) {
       q.variant = pick(q);
     }
-    *bytes += q.g.L * q.g.rows;
-    rs->push_back(q);
-    where->push_back(i);
+    out->bytes += q.g.L * q.g.rows;
+    out->rs.push_back(q);
+    out->where.push_back(i);
   }
   return TEMPI_SUCCESS;
 }
@@ -647,12 +698,11 @@ bool saturated(const std::vector<Req> &rs) {
 
 // gives the requests whose variant was left to the library `pick`'s
 template <class Pick>
-void repick(const tempi_batch_request *reqs, const std::vector<int64_t> &where,
-            std::vector<Req> *rs, Pick &&pick) {
-  for (size_t k = 0; k < rs->size(); ++k) {
-    const int asked = reqs[where[k]].variant;
+void repick(const tempi_batch_request *reqs, Resolved *q, Pick &&pick) {
+  for (size_t k = 0; k < q->rs.size(); ++k) {
+    const int asked = reqs[q->where[k]].variant;
     if (asked < 0 || asked >= kNumVariants) {
-      (*rs)[k].variant = pick((*rs)[k]);
+      q->rs[k].variant = pick(q->rs[k]);
     }
   }
 }
@@ -684,8 +734,8 @@ TEMPI_EXPORT int tempi_batch_create(const tempi_batch_request *reqs, int64_t n,
   tempi_batch *b = owner.get();
   b->requests = n;
   b->variants.assign((size_t)n, -1);
-  std::vector<Req> rs;
-  std::vector<int64_t> where;
+  Resolved q;
+  std::vector<Req> &rs = q.rs;
   // the per-copy policy first (in small batches the learned selector's
   // picks for requests under 1 MiB ran the faces of 128^3 - 256^3 float
   // grids 5-28 % faster than the closed-form rule's), then the batch rule
@@ -693,33 +743,33 @@ TEMPI_EXPORT int tempi_batch_create(const tempi_batch_request *reqs, int64_t n,
   // selector evaluates all the batch's new shapes in one inference first:
   // one launch per shape took 0.14 s to create the 4 096-request batch.
   int err = resolve_requests(
-      reqs, n, [](const Req &) { return -1; }, &rs, &where, &b->bytes);
+      reqs, n, true, device_buffers, [](const Req &) { return -1; }, &q);
   if (err) {
     return err;
   }
+  b->bytes = q.bytes;
   if (method == TEMPI_SELECT_MODEL ||
       (method == TEMPI_SELECT_DEFAULT && model_available())) {
     std::vector<CopyShape> shapes;
-    for (const Req &q : rs) {
-      if (q.variant < 0) {
-        shapes.push_back({q.g, q.ds, q.dp, q.dir});
+    for (const Req &r : rs) {
+      if (r.variant < 0) {
+        shapes.push_back({r.g, r.ds, r.dp, r.dir});
       }
     }
     model_prefetch(shapes);
   }
-  for (Req &q : rs) {
-    if (q.variant < 0) {
-      q.variant = choose(q.g, q.ds, q.dp, q.dir, method, library_stream(),
+  for (Req &r : rs) {
+    if (r.variant < 0) {
+      r.variant = choose(r.g, r.ds, r.dp, r.dir, method, library_stream(),
                          CopyUse::kInBatch)
                       .variant;
     }
   }
   if (method == TEMPI_SELECT_DEFAULT && saturated(rs)) {
-    repick(reqs, where, &rs,
-           [](const Req &q) { return saturated_variant(q.g, q.dir); });
+    repick(reqs, &q, [](const Req &r) { return saturated_variant(r.g, r.dir); });
   }
   for (size_t k = 0; k < rs.size(); ++k) {
-    b->variants[(size_t)where[k]] = rs[k].variant;
+    b->variants[(size_t)q.where[k]] = rs[k].variant;
   }
   if ((err = build_batch(b, rs))) {
     return err;
@@ -1007,49 +1057,55 @@ int scratch_slot(ScratchSlot **out) {
 } // namespace
 } // namespace tempi
 
+namespace {
+
+// The variants and tables of tempi_batch_run_noalloc.  The closed-form rule:
+// the learned selector and trial timings would allocate device memory on
+// first use.
+template <class Buffers>
+int plan_noalloc(const tempi_batch_request *reqs, int64_t n, bool on_device,
+                 Buffers &&buffers, Resolved *q, BatchPlan *pl) {
+  int err = resolve_requests(
+      reqs, n, on_device, buffers,
+      [](const Req &r) { return heuristic_variant(r.g, r.ds, r.dp, r.dir); }, q);
+  if (err || q->rs.empty()) {
+    return err;
+  }
+  if (saturated(q->rs)) {
+    repick(reqs, q, [](const Req &r) { return saturated_variant(r.g, r.dir); });
+  }
+  if ((err = plan_batch(q->rs, pl))) {
+    return err;
+  }
+  if (pl->image.size() > kScratchBytes) {
+    // as many rows to a tile record as a kernel moves
+    for (Req &r : q->rs) {
+      r.wide = true;
+    }
+    repick(reqs, q, fewest_tiles);
+    err = plan_batch(q->rs, pl);
+  }
+  return err;
+}
+
+} // namespace
+
 TEMPI_EXPORT int tempi_batch_run_noalloc(const tempi_batch_request *reqs,
                                          int64_t n, void *stream) {
   if ((n > 0 && !reqs) || n < 0) {
     return set_error(TEMPI_ERR_ARG, "bad argument");
   }
-  std::vector<Req> rs;
-  std::vector<int64_t> where;
-  int64_t bytes = 0;
-  // the closed-form rule: the learned selector and trial timings would
-  // allocate device memory on first use
-  int err = resolve_requests(
-      reqs, n,
-      [](const Req &q) { return heuristic_variant(q.g, q.ds, q.dp, q.dir); },
-      &rs, &where, &bytes);
-  if (err) {
-    return err;
-  }
-  if (rs.empty()) {
-    return TEMPI_SUCCESS;
-  }
-  if (saturated(rs)) {
-    repick(reqs, where, &rs,
-           [](const Req &q) { return saturated_variant(q.g, q.dir); });
-  }
+  Resolved q;
   BatchPlan pl;
-  if ((err = plan_batch(rs, &pl))) {
+  int err = plan_noalloc(reqs, n, true, device_buffers, &q, &pl);
+  if (err || q.rs.empty()) {
     return err;
-  }
-  if (pl.image.size() > kScratchBytes) {
-    // as many rows to a tile record as a kernel moves
-    for (Req &q : rs) {
-      q.wide = true;
-    }
-    repick(reqs, where, &rs, fewest_tiles);
-    if ((err = plan_batch(rs, &pl))) {
-      return err;
-    }
   }
   if (pl.image.size() > kScratchBytes) {
     return set_error(TEMPI_ERR_UNSUPPORTED,
                      "batch tables of %zu B (%zu requests, %u tiles) exceed "
                      "the %zu B of static scratch",
-                     pl.image.size(), rs.size(), pl.launch.ntiles,
+                     pl.image.size(), q.rs.size(), pl.launch.ntiles,
                      kScratchBytes);
   }
   ScratchSlot *sl = nullptr;
@@ -1069,5 +1125,86 @@ TEMPI_EXPORT int tempi_batch_run_noalloc(const tempi_batch_request *reqs,
   launch_kernel(placed(pl, sl->ptr), s);
   TEMPI_HIP_CHECK(hipGetLastError());
   ++counters().batch_launches;
+  return TEMPI_SUCCESS;
+}
+
+// What tempi_batch_run_noalloc would launch for requests whose addresses are
+// numbers: the same plan, read back from the tables' host image.
+TEMPI_EXPORT int tempi_batch_emulate(const tempi_batch_request *reqs, int64_t n,
+                                     int packed_on_host, int32_t *variants,
+                                     tempi_batch_emulation *out) {
+  if ((n > 0 && !reqs) || n < 0 || !out) {
+    return set_error(TEMPI_ERR_ARG, "bad argument");
+  }
+  *out = tempi_batch_emulation{};
+  Resolved q;
+  BatchPlan pl;
+  const int err = plan_noalloc(
+      reqs, n, false,
+      [&](const tempi_batch_request &r, Req *rq) {
+        rq->ds = static_cast<const char *>(r.strided);
+        rq->dp = static_cast<char *>(r.packed);
+        rq->g.host = packed_on_host != 0;
+        return true;
+      },
+      &q, &pl);
+  if (err) {
+    return err;
+  }
+  if (variants) {
+    std::fill(variants, variants + n, -1);
+    for (size_t k = 0; k < q.rs.size(); ++k) {
+      variants[q.where[k]] = q.rs[k].variant;
+    }
+  }
+  out->requests = (int64_t)q.rs.size();
+  out->fits_static_tables = pl.image.size() <= kScratchBytes;
+  if (q.rs.empty()) {
+    out->exact = 1;
+    return TEMPI_SUCCESS;
+  }
+  const BatchLaunch &L = pl.launch;
+  out->tiles = L.ntiles;
+  out->grid = L.grid;
+  const BatchItem *items = reinterpret_cast<const BatchItem *>(pl.image.data());
+  std::vector<uint64_t> first(q.rs.size() + 1, 0);
+  for (size_t r = 0; r < q.rs.size(); ++r) {
+    first[r + 1] = first[r] + items[r].ntiles;
+  }
+  std::vector<uint8_t> runs(first.back(), 0);
+  bool inside = true;
+  const auto run = [&](uint32_t xcd, uint32_t r, uint32_t l) {
+    if (r >= q.rs.size() || l >= items[r].ntiles) {
+      inside = false;
+      return;
+    }
+    const Geom &g = q.rs[r].g;
+    runs[first[r] + l] += runs[first[r] + l] < 2;
+    ++out->xcd_tiles[xcd];
+    out->xcd_bytes[xcd] +=
+        ((double)touched_bytes(g) + (double)g.L * g.rows) / items[r].ntiles;
+  };
+  if (L.small) {
+    for (uint32_t r = 0; r < L.ix.n; ++r) {
+      for (uint32_t k = 0; k < kXcds * L.ix.share[r]; ++k) {
+        const uint32_t l = k % kXcds * L.ix.share[r] + k / kXcds;
+        if (l < L.ix.ntiles[r]) {
+          run((L.ix.base[r] + k) % kXcds, r, l);
+        }
+      }
+    }
+  } else {
+    const Tile *tiles = reinterpret_cast<const Tile *>(pl.image.data() + pl.tl_off);
+    const uint32_t *begin =
+        reinterpret_cast<const uint32_t *>(pl.image.data() + pl.xb_off);
+    for (uint32_t x = 0; x < (L.xcd_split ? kXcds : 1u); ++x) {
+      const uint32_t end = L.xcd_split ? begin[x + 1] : L.ntiles;
+      for (uint32_t t = L.xcd_split ? begin[x] : 0; t < end; ++t) {
+        run(L.xcd_split ? x : t % kXcds, tiles[t].item, tiles[t].tile);
+      }
+    }
+  }
+  out->exact = inside && std::all_of(runs.begin(), runs.end(),
+                                     [](uint8_t c) { return c == 1; });
   return TEMPI_SUCCESS;
 }

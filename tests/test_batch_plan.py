@@ -1,0 +1,84 @@
+"""The tile plan of a batch, on the host: every tile of every request runs
+exactly once, and each of the eight XCDs gets an eighth of the traffic (to one
+tile) wherever the requests' buffers lie."""
+import random
+
+import pytest
+
+import tempi_amd as ta
+
+GIB = 1 << 30
+
+
+def rows2d(length, rows, stride, start=0):
+    return ta.StridedBlock.make(start, start + max(rows * abs(stride), length), [length, rows],
+                                [1, stride])
+
+
+def far_grids(gap):
+    """52 requests on two grids of 20 MiB: 26 faces of 40 tiles each."""
+    sb = rows2d(512, 1280, 600)
+    return [(sb, (1 << 40) + g * gap + k * (20 << 20) // 26, (1 << 45) + k * GIB, 1, ta.DIR_PACK)
+            for g in (0, 1) for k in range(26)]
+
+
+def one_window():
+    """100 packs of the same 4 KiB, sixteen times over (stride 0)."""
+    sb = rows2d(4096, 16, 0)
+    return [(sb, 1 << 40, (1 << 45) + (k << 20), 1, ta.DIR_PACK) for k in range(100)]
+
+
+def same_face():
+    sb = rows2d(2048, 512, 4096)
+    return [(sb, 1 << 40, (1 << 45) + (k << 20), 1, ta.DIR_PACK) for k in range(26)]
+
+
+def sparse_and_dense():
+    """One request across 256 GiB, the others close together inside it."""
+    reqs = [(rows2d(64, 1 << 12, 1 << 26), 1 << 40, 1 << 45, 1, ta.DIR_PACK)]
+    sb = rows2d(256, 4096, 320)
+    return reqs + [(sb, (1 << 40) + 100 * GIB + (k << 20) * 2, (1 << 46) + (k << 20), 1,
+                    ta.DIR_UNPACK) for k in range(60)]
+
+
+def mixed():
+    rng = random.Random(7)
+    reqs = []
+    for k in range(300):
+        length = rng.choice((1, 4, 12, 24, 100, 512, 4096))
+        rows = rng.randint(1, 3000)
+        stride = rng.choice((length, length + rng.randint(1, 500), -(length + 64)))
+        start = rows * abs(stride) if stride < 0 else 0
+        at = (1 << 40) + rng.randrange(1 << rng.choice((20, 30, 38)))
+        reqs.append((rows2d(length, rows, stride, start), at, (1 << 46) + (k << 24), 1,
+                     rng.choice((ta.DIR_PACK, ta.DIR_UNPACK))))
+    return reqs
+
+
+# bound of one tile's bytes: 1024 rows of a line each, both sides
+LARGEST_TILE = 1024 * (128 + 128) + 2 * 65536
+
+
+@pytest.mark.parametrize("make", [
+    lambda: far_grids(16 * GIB), lambda: far_grids(100 * GIB), lambda: far_grids(-(1 << 39)),
+    one_window, same_face, sparse_and_dense, mixed,
+], ids=["16GiB", "100GiB", "below", "one_window", "same_face", "sparse", "mixed"])
+def test_every_xcd_gets_its_share(make):
+    reqs = make()
+    e = ta.batch_emulate(reqs)
+    assert e["exact"] == 1 and e["requests"] == len(reqs)
+    assert sum(e["xcd_tiles"]) == e["tiles"] >= 64
+    assert e["grid"] == 8 * max(e["xcd_tiles"])
+    total = sum(e["xcd_bytes"])
+    assert max(e["xcd_bytes"]) <= total / 8 + LARGEST_TILE
+    assert min(e["xcd_bytes"]) >= total / 8 - LARGEST_TILE
+
+
+@pytest.mark.parametrize("n", [1, 8, 9])
+def test_few_requests(n):
+    for rows in (1, 2, 63, 1000):
+        reqs = [(rows2d(12, rows, 24), (1 << 40) + (k << 30), (1 << 45) + (k << 20), 1,
+                 ta.DIR_UNPACK) for k in range(n)]
+        e = ta.batch_emulate(reqs)
+        assert e["exact"] == 1 and sum(e["xcd_tiles"]) == e["tiles"]
+    assert ta.batch_emulate([])["exact"] == 1
