@@ -280,7 +280,9 @@ int tempi_launch_latency_us(int reps, float *host_us, float *device_us);
    request that leaves it to the library (variant -1), as for a single copy
    of that request; under the default policy a batch of more than 8 requests
    and 8 tiles per CU picks by row length, direction and where the packed
-   bytes are. */
+   bytes are.  A request of 2^31 work units or more with that pick takes a
+   variant of longer units (so does one that names 12, 16 or 17, whose units
+   are the shortest); what none holds is refused (TEMPI_ERR_UNSUPPORTED). */
 typedef struct tempi_batch_request {
   tempi_strided_block sb; /* layout of one object                          */
   const void *strided;    /* strided buffer origin (pack: in, unpack: out)  */

@@ -627,12 +627,50 @@ int build_batch(tempi_batch *b, const std::vector<Req> &rs) {
 // Tiles of a resolved request (one workgroup pass each) in a batch of more
 // than kSmallItems.
 uint64_t tiles_of(const Req &q) {
-  const VariantDesc &v = kVariants[q.variant];
-  const int64_t per_unit = (int64_t)v.P * v.U;
-  const int64_t nseg = std::max<int64_t>(1, (q.g.L / v.W + per_unit - 1) / per_unit);
-  const uint64_t units = (uint64_t)(q.g.rows * nseg);
-  const uint64_t per_tile = units_per_tile(v, q.wide);
+  const uint64_t units = (uint64_t)units_of(q.g, q.variant);
+  const uint64_t per_tile = units_per_tile(kVariants[q.variant], q.wide);
   return (units + per_tile - 1) / per_tile;
+}
+
+bool fits(const Req &q, int variant) {
+  return units_of(q.g, variant) < kMaxUnits;
+}
+
+// of the variants that hold a request, the one that splits it into the fewest
+// tiles
+int fewest_tiles(const Req &q) {
+  Req r = q;
+  uint64_t best = UINT64_MAX;
+  int variant = q.variant;
+  for (r.variant = 0; r.variant < kNumVariants; ++r.variant) {
+    const uint64_t t = tiles_of(r);
+    if (t < best && fits(q, r.variant)) {
+      best = t;
+      variant = r.variant;
+    }
+  }
+  return variant;
+}
+
+// the kernel like `variant` whose units are longer than 12 B or 32 B of a row
+int wider(int variant) {
+  return variant == 12 ? 7 : variant == 16 ? 13 : variant == 17 ? 15 : variant;
+}
+
+// A request is not split, so its units have to stay below kMaxUnits, and the
+// rules pick by speed whatever the size: rows of host memory, as units of
+// 16 B, reach the limit at 32 GiB.  Returns q.variant or, where it does not
+// hold the request, the closed-form rule's or the one of fewest tiles; for a
+// variant the caller asked for, the wider one like it.
+int fitting_variant(const Req &q, bool asked) {
+  if (fits(q, q.variant)) {
+    return q.variant;
+  }
+  if (asked) {
+    return wider(q.variant);
+  }
+  const int rule = heuristic_variant(q.g, q.ds, q.dp, q.dir);
+  return fits(q, rule) ? rule : fewest_tiles(q);
 }
 
 // The default policy's rule for batches with more tiles than the grid runs at
@@ -696,30 +734,25 @@ bool saturated(const std::vector<Req> &rs) {
   return tiles > (uint64_t)device_cu_count() * 8;
 }
 
+bool asked_for(const tempi_batch_request &r) {
+  return r.variant >= 0 && r.variant < kNumVariants;
+}
+
 // gives the requests whose variant was left to the library `pick`'s
 template <class Pick>
 void repick(const tempi_batch_request *reqs, Resolved *q, Pick &&pick) {
   for (size_t k = 0; k < q->rs.size(); ++k) {
-    const int asked = reqs[q->where[k]].variant;
-    if (asked < 0 || asked >= kNumVariants) {
+    if (!asked_for(reqs[q->where[k]])) {
       q->rs[k].variant = pick(q->rs[k]);
     }
   }
 }
 
-// the variant that splits a request into the fewest tiles
-int fewest_tiles(const Req &q) {
-  Req r = q;
-  uint64_t best = UINT64_MAX;
-  int variant = q.variant;
-  for (r.variant = 0; r.variant < kNumVariants; ++r.variant) {
-    const uint64_t t = tiles_of(r);
-    if (t < best) {
-      best = t;
-      variant = r.variant;
-    }
+void fit_variants(const tempi_batch_request *reqs, Resolved *q) {
+  for (size_t k = 0; k < q->rs.size(); ++k) {
+    Req &r = q->rs[k];
+    r.variant = fitting_variant(r, asked_for(reqs[q->where[k]]));
   }
-  return variant;
 }
 
 } // namespace
@@ -768,6 +801,7 @@ TEMPI_EXPORT int tempi_batch_create(const tempi_batch_request *reqs, int64_t n,
   if (method == TEMPI_SELECT_DEFAULT && saturated(rs)) {
     repick(reqs, &q, [](const Req &r) { return saturated_variant(r.g, r.dir); });
   }
+  fit_variants(reqs, &q);
   for (size_t k = 0; k < rs.size(); ++k) {
     b->variants[(size_t)q.where[k]] = rs[k].variant;
   }
@@ -1074,6 +1108,7 @@ int plan_noalloc(const tempi_batch_request *reqs, int64_t n, bool on_device,
   if (saturated(q->rs)) {
     repick(reqs, q, [](const Req &r) { return saturated_variant(r.g, r.dir); });
   }
+  fit_variants(reqs, q);
   if ((err = plan_batch(q->rs, pl))) {
     return err;
   }
@@ -1081,6 +1116,9 @@ int plan_noalloc(const tempi_batch_request *reqs, int64_t n, bool on_device,
     // as many rows to a tile record as a kernel moves
     for (Req &r : q->rs) {
       r.wide = true;
+      if (r.variant != 12) { // four of its units to a lane are as many rows
+        r.variant = wider(r.variant);
+      }
     }
     repick(reqs, q, fewest_tiles);
     err = plan_batch(q->rs, pl);

@@ -333,6 +333,9 @@ constexpr bool nt_loads(Nontemporal nt, int dir) {
 // copy along its outer row dimensions.
 constexpr int64_t kMaxUnits = 1ll << 31;
 
+// work units of a copy with `variant`
+int64_t units_of(const Geom &g, int variant);
+
 // Fill the kernel parameters of one copy with `variant`; `whole`: its rows
 // are whole words.  A copy of kMaxUnits units or more is reported as
 // TEMPI_ERR_UNSUPPORTED.

@@ -465,6 +465,10 @@ static int64_t segments_of(const Geom &g, int variant) {
   return std::max<int64_t>(1, (g.L / v.W + per_unit - 1) / per_unit);
 }
 
+int64_t units_of(const Geom &g, int variant) {
+  return g.rows * segments_of(g, variant);
+}
+
 // Call piece(geometry, strided, packed) for each launch of a copy: rows
 // longer than 1 GiB go as 1 GiB pieces, and a copy of kMaxUnits units or
 // more is cut along its outer row dimensions -- a run of whole indices of
@@ -730,7 +734,7 @@ bool on_library_device() {
 // one launch of at most kSignalMaxBlocks workgroups, on the library
 // stream's device
 bool signal_fits(const Geom &g, int variant, int max_blocks) {
-  const int64_t units = g.rows * segments_of(g, variant);
+  const int64_t units = units_of(g, variant);
   return g.L <= (1ll << 30) && units < kMaxUnits &&
          grid_of(variant, (uint32_t)units, max_blocks, device_cu_count()) <=
              kSignalMaxBlocks &&

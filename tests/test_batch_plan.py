@@ -82,3 +82,57 @@ def test_few_requests(n):
         e = ta.batch_emulate(reqs)
         assert e["exact"] == 1 and sum(e["xcd_tiles"]) == e["tiles"]
     assert ta.batch_emulate([])["exact"] == 1
+
+
+# -- what a batch takes ---------------------------------------------------------
+#
+# Sizes whose work units would reach 2^31 with the variant that is fastest:
+# the plan takes one that holds them.  (No table of these sizes fits the static
+# array, which the plan reports and does not refuse.)
+
+SMALL = [(rows2d(64, 64, 128), (1 << 40) + (k << 20), (1 << 44) + (k << 20), 1, ta.DIR_PACK)
+         for k in range(12)]
+
+
+def plan_of_large(length, rows, direction, host=False, variant=-1):
+    large = (rows2d(length, rows, length + 8), 1 << 46, 1 << 47, 1, direction, variant)
+    e = ta.batch_emulate(SMALL + [large], packed_on_host=host)
+    assert e["exact"] == 1 and e["requests"] == len(SMALL) + 1
+    return e
+
+
+@pytest.mark.parametrize("length,rows,direction,host", [
+    (4096, 1 << 23, ta.DIR_PACK, True),    # 32 GiB in 4-KiB rows of host memory
+    (4096, 1 << 23, ta.DIR_UNPACK, True),
+    (40, 1 << 30, ta.DIR_UNPACK, False),   # 40-B rows: two units of 32 B
+    (100, 1 << 29, ta.DIR_PACK, True),
+])
+def test_large_requests_are_taken(length, rows, direction, host):
+    plan_of_large(length, rows, direction, host)
+
+
+@pytest.mark.parametrize("variant,length,rows", [
+    (12, 24, 1 << 30), (16, 48, 1 << 29), (17, 64, 1 << 30),
+])
+def test_large_requests_of_a_given_variant_are_taken(variant, length, rows):
+    plan_of_large(length, rows, ta.DIR_PACK, variant=variant)
+
+
+def test_rows_beyond_the_limit_stay_refused():
+    for host in (False, True):
+        with pytest.raises(ta.TempiError):
+            plan_of_large(16, 1 << 31, ta.DIR_PACK, host)
+    for variant in (7, 9, 12, 16, 17):
+        with pytest.raises(ta.TempiError):
+            plan_of_large(16, 1 << 31, ta.DIR_PACK, variant=variant)
+
+
+@pytest.mark.parametrize("variant", [-1, 0, 1, 2, 3, 4, 5, 6, 7, 13, 14, 15, 16, 17])
+def test_static_tables_hold_large_batches(variant):
+    """7.5 GiB in 4-KiB rows are 480 Ki tiles of 16 KiB: they fit the static
+    tables with each variant whose tiles are that large, and with 16 and 17,
+    which give way to one of them."""
+    reqs = [(rows2d(4096, 160 << 10, 4160), (1 << 40) + (k << 30), (1 << 44) + (k << 30), 1,
+             ta.DIR_PACK, variant) for k in range(12)]
+    e = ta.batch_emulate(reqs)
+    assert e["exact"] == 1 and e["fits_static_tables"] == 1
