@@ -598,22 +598,39 @@ int launch_copy(const Geom &g, const char *strided, char *packed, int dir,
 // MPI_Pack and MPI_Unpack return when their copy is done.  On MI355X an
 // empty kernel's own store reaches the host 5.7 us after its launch begins,
 // but hipStreamSynchronize returns after 11.1 us: the rest is the runtime's
-// end-of-kernel processing.  A copy of one launch of at most
-// kSignalMaxBlocks workgroups on the library stream therefore signals its
-// own completion (KParams::signal) and the host spins on the flag.  In larger
-// grids each workgroup's release writes its XCD's L2 back and those queue
-// behind each other (counting in 32 leaves instead of one counter changes
-// nothing), so a one-thread kernel behind the copy stores the flag instead: it
-// starts after the copy's own end-of-kernel write-back.  Copies of 16 KiB per
-// workgroup, launch to the host seeing it, us:
+// end-of-kernel processing.  A copy of one launch of few workgroups on the
+// library stream therefore signals its own completion (KParams::signal) and
+// the host spins on the flag.  In larger grids each workgroup's release writes
+// its XCD's L2 back and those queue behind each other (counting in 32 leaves
+// instead of one counter changes nothing), so a one-thread kernel behind the
+// copy stores the flag instead: it starts after the copy's own end-of-kernel
+// write-back.  Contiguous copies of 16 KiB per workgroup, launch to the host
+// seeing it, us:
 //   workgroups               64    128    256    512   1024   2048
 //   own signal              8.9   10.7   14.3   21.9   37.2   72.1
 //   signal kernel behind    9.9   10.0   10.2   10.8   11.2   17.2
 //   hipStreamSynchronize   11.9   12.2   12.5   13.4   14.5   20.8
+//
+// How few depends on what a write-back finds.  Where the lanes of a row's
+// group store next to each other, whole lines; where each lane stores a row of
+// its own, lines of which the rest is still to come, and in host memory each
+// of those is a write over the link by itself.  Own signal less signal kernel,
+// us, median (most) over rows of 4 B - 1 KiB 100 B apart, MPI_Pack and
+// MPI_Unpack:
+//   workgroups                       16           32           64          128
+//   packed on the device, P > 1  -0.7 (-0.4)  -0.5 (-0.2)  -0.3 (0.5)   0.9 (2.7)
+//                         P = 1  -0.6 (0.1)   -0.2 (0.5)    0.5 (1.3)   2.2 (3.3)
+//   packs to the host,    P > 1  -0.8 (0.4)   -0.6 (0.1)   -0.3 (0.5)   0.2 (2.6)
+//                         P = 1  -0.5 (1.0)    1.0 (3.0)    4.4 (15)     15 (44)
+//   unpacks from it,      P > 1  -0.4 (0.4)   -0.2 (0.9)    0.2 (1.6)   2.2 (3.2)
+//                         P = 1  -0.2 (0.5)    0.2 (0.9)    1.0 (1.9)   2.9 (3.7)
 
 namespace {
 
-constexpr int64_t kSignalMaxBlocks = 128;
+// most workgroups of a copy that signals for itself
+int64_t own_signal_blocks(const Geom &g, int variant) {
+  return kVariants[variant].P > 1 ? 64 : g.host ? 16 : 48;
+}
 
 struct SignalState {
   std::mutex mu; // held from a signal's number to its launch
@@ -731,13 +748,12 @@ bool on_library_device() {
   return hipSuccess == hipGetDevice(&dev) && dev == library_device();
 }
 
-// one launch of at most kSignalMaxBlocks workgroups, on the library
-// stream's device
+// one launch of few enough workgroups, on the library stream's device
 bool signal_fits(const Geom &g, int variant, int max_blocks) {
   const int64_t units = units_of(g, variant);
   return g.L <= (1ll << 30) && units < kMaxUnits &&
          grid_of(variant, (uint32_t)units, max_blocks, device_cu_count()) <=
-             kSignalMaxBlocks &&
+             own_signal_blocks(g, variant) &&
          on_library_device();
 }
 

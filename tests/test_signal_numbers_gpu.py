@@ -63,3 +63,45 @@ def test_an_unread_error_of_the_application(mpi, rows, block, stride):
         assert lib.hipGetLastError() == INVALID_DEVICE  # still the application's
     mpi.free(hb)
     mpi.free(hs)
+
+
+@pytest.mark.parametrize("block,rows,mapped,own", [
+    (24, 21845, True, False),   # 512 KiB of lane-per-row stores over the link
+    (100, 13107, True, False),  # 1.25 MiB in 103 workgroups of four lanes a row
+    (24, 4096, True, True),     # 96 KiB in 16 workgroups
+    (256, 1024, True, True),    # 32 workgroups, whole lines
+    (256, 1024, False, True),
+    (12, 21845, False, None),   # either, by the pick
+    (4096, 8192, True, False),  # 32 MiB
+])
+def test_the_copy_signals_itself_where_that_is_the_shorter_wait(mpi, block, rows, mapped, own):
+    """... and its bytes are there, in mapped memory for the host itself to
+    read, when the call returns."""
+    spec = ("vector", rows, block, block + 100, tc.BYTE)
+    h = mpi.type_from_spec(spec)
+    o = orc.OracleType(spec)
+    n, size = o.span(1)[1], o.size()
+    src, dst = ta.DeviceBuffer(n), ta.DeviceBuffer(n)
+    packed = ta.DeviceBuffer(size, mapped=mapped)
+    lib = hip()
+    for it in range(20 if size < (1 << 21) else 3):
+        host = orc.splitmix_bytes(n, 300 + it)
+        want = o.pack(host, 0, 1)
+        src.upload(host)
+        dst.fill(0xAB)
+        n0, k0 = ta.signals()
+        assert mpi.pack(src.addr(), 1, h, packed.addr(), size) == (0, size)
+        if mapped:
+            got = np.ctypeslib.as_array((ctypes.c_uint8 * size).from_address(packed.addr()))
+        else:
+            got = fetch(lib, packed, size)
+        assert (got == want).all(), it
+        n1, k1 = ta.signals()
+        assert n1 - n0 == 1
+        if own is not None:
+            assert k1 - k0 == (0 if own else 1)
+        assert mpi.unpack(packed.addr(), size, dst.addr(), 1, h) == (0, size)
+        ref = np.full(n, 0xAB, np.uint8)
+        o.unpack(want, ref, 0, 1)
+        assert (fetch(lib, dst, n) == ref).all(), it
+    mpi.free(h)
