@@ -365,16 +365,19 @@ Choice choose(const Geom &g, const char *strided, char *packed, int dir,
               int method, hipStream_t stream, CopyUse use) {
   const bool in_place = use == CopyUse::kNext;
   Choice c;
-  if (method == TEMPI_SELECT_DEFAULT && use != CopyUse::kInBatch &&
-      (c.variant = latency_variant(g)) >= 0) {
-    return c;
-  }
   // in batches the packs' picks reach the link as well as the rule's (three
   // faces of a 512^3 float grid to mapped memory 175 us, 178 by the rule), the
   // unpacks' do not (192 us, 174 by the rule)
   if (method == TEMPI_SELECT_DEFAULT && g.host &&
       (use != CopyUse::kInBatch || dir == TEMPI_DIR_UNPACK) &&
       (c.variant = link_variant(g, dir)) >= 0) {
+    return c;
+  }
+  // after the link: of 512 KiB to 1 MiB its rule is the better one
+  // (MPI_Unpack of 1 MiB from mapped memory, rows of 64 B - 4 KiB: 28.8-29.2 us
+  // by the link's variant, 33.3-36.2 by this one)
+  if (method == TEMPI_SELECT_DEFAULT && use != CopyUse::kInBatch &&
+      (c.variant = latency_variant(g)) >= 0) {
     return c;
   }
   c.variant = heuristic_variant(g, strided, packed, dir);
