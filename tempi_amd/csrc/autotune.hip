@@ -361,6 +361,16 @@ static int verify_candidates(const Geom &g, const char *strided, char *packed,
   return TEMPI_SUCCESS;
 }
 
+// The timed candidates follow from the shape and, in unpacks, from whether
+// rows cut 64-B sectors of the strided side (streamed_variant): the shape's
+// key, which has that side's address modulo 16 only, and that.
+static std::string verify_key_of(const std::string &shape, const Geom &g,
+                                 const char *strided, int dir) {
+  const bool sectors = dir == TEMPI_DIR_UNPACK &&
+                       geom_aligned(g, strided, strided + g.start, 64);
+  return shape + (sectors ? 's' : 'c');
+}
+
 Choice choose(const Geom &g, const char *strided, char *packed, int dir,
               int method, hipStream_t stream, CopyUse use) {
   const bool in_place = use == CopyUse::kNext;
@@ -384,10 +394,13 @@ Choice choose(const Geom &g, const char *strided, char *packed, int dir,
   if (method == TEMPI_SELECT_MODEL ||
       (method == TEMPI_SELECT_DEFAULT && model_available())) {
     const std::string key = shape_key_of(g, strided, packed, dir);
-    if (method == TEMPI_SELECT_DEFAULT && times_cold(g)) {
+    // (a batch's pack to host memory is not timed: the trial's scratch is
+    // device memory)
+    if (method == TEMPI_SELECT_DEFAULT && times_cold(g) && !g.host) {
+      const std::string vkey = verify_key_of(key, g, strided, dir);
       {
         std::lock_guard<std::mutex> lk(g_tune_mu);
-        auto it = g_verify_cache.find(key);
+        auto it = g_verify_cache.find(vkey);
         if (it != g_verify_cache.end()) {
           return it->second;
         }
@@ -396,14 +409,18 @@ Choice choose(const Geom &g, const char *strided, char *packed, int dir,
       if (stream && !verify_candidates(g, strided, packed, dir, c.variant,
                                        stream, in_place, &v)) {
         std::lock_guard<std::mutex> lk(g_tune_mu);
-        g_verify_cache[key] = v;
+        g_verify_cache[vkey] = v;
         return v;
       }
     }
     const int v = model_variant(g, strided, packed, dir, key);
     if (v >= 0) {
       // requests of a batch share lines with each other (a halo's faces,
-      // edges and corners): nontemporal loads would read those again
+      // edges and corners): nontemporal loads would read those again.  Those
+      // timed above, of 64 MiB and more, are large enough to be streamed all
+      // the same (pack + unpack batches of four requests of 64-B rows, 64 MiB
+      // each: 300 us cached, 212 streamed; three faces 16 cells deep of an
+      // 832^3 float grid 125 and 92)
       c.variant =
           method == TEMPI_SELECT_DEFAULT
               ? streamed_variant(v, g, strided, dir,
