@@ -54,6 +54,7 @@ void read_environment() {
   Env &e = env();
   e.disable = nullptr != std::getenv("TEMPI_DISABLE");
   e.no_pack = nullptr != std::getenv("TEMPI_NO_PACK");
+  e.no_signal = nullptr != std::getenv("TEMPI_NO_SIGNAL");
   e.no_type_commit = nullptr != std::getenv("TEMPI_NO_TYPE_COMMIT");
   if (const char *s = std::getenv("TEMPI_SELECT")) {
     if (0 == strcmp(s, "heuristic")) {

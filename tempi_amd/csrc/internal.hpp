@@ -73,6 +73,7 @@ inline int check_direction(int dir) {
 struct Env {
   bool disable = false;        // TEMPI_DISABLE: pure pass-through
   bool no_pack = false;        // TEMPI_NO_PACK: MPI_Pack/Unpack -> library
+  bool no_signal = false; // TEMPI_NO_SIGNAL: copies are waited for by the runtime
   bool no_type_commit = false; // TEMPI_NO_TYPE_COMMIT: no canonicalization
   // TEMPI_DATATYPE_{ONESHOT,DEVICE,STAGED,AUTO}: how non-contiguous device
   // data is sent (TEMPI_METHOD_*; UNKNOWN = choose by the system model)
@@ -248,11 +249,15 @@ int launch_copy_signalled(const Geom &g, const char *strided, char *packed,
 // is done; 0: there is none
 unsigned long long signal_stream();
 bool signal_reached(unsigned long long seq);
-// has signal `seq` arrived (0: is the library stream done)?  `polls` counts
-// the caller's calls
-int poll_signal_or_stream(unsigned long long seq, uint32_t *polls, bool *done);
-// until signal `seq` arrives (0: until the library stream is done)
-int wait_signal_or_stream(unsigned long long seq);
+// an event behind the library stream's work so far, for a request that has no
+// signal (null: there is none, and it waits for the whole stream)
+hipEvent_t mark_library_stream();
+// has signal `seq` arrived (0: `ev`, or if null the library stream)?  `polls`
+// counts the caller's calls
+int poll_signal_or_stream(unsigned long long seq, hipEvent_t ev,
+                          uint32_t *polls, bool *done);
+// until signal `seq` arrives (0: `ev`, or if null the library stream)
+int wait_signal_or_stream(unsigned long long seq, hipEvent_t ev = nullptr);
 // until everything on the library stream is done
 int wait_library_stream();
 

@@ -674,6 +674,9 @@ bool signal_ready(SignalState &st) {
     return st.flag != nullptr && !st.off.load(std::memory_order_relaxed);
   }
   st.tried = true;
+  if (env().no_signal) {
+    return false;
+  }
   // the counter is zeroed on the library stream (which does not wait for the
   // null stream) before the first signalled launch
   hipStream_t s = library_stream();
@@ -823,14 +826,29 @@ bool signal_reached(unsigned long long seq) {
   return seq && st.flag && flag_at(st, seq);
 }
 
-int poll_signal_or_stream(unsigned long long seq, uint32_t *polls, bool *done) {
+hipEvent_t mark_library_stream() {
+  hipEvent_t ev = nullptr;
+  if (hipSuccess == hipEventCreateWithFlags(&ev, hipEventDisableTiming) &&
+      hipSuccess == hipEventRecord(ev, library_stream())) {
+    return ev;
+  }
+  (void)hipGetLastError(); // one of these two calls'
+  if (ev) {
+    (void)hipEventDestroy(ev);
+  }
+  return nullptr;
+}
+
+int poll_signal_or_stream(unsigned long long seq, hipEvent_t ev,
+                          uint32_t *polls, bool *done) {
   *done = signal_reached(seq);
   // a signal that does not come is looked after in the stream's own state,
   // every so many polls: the query costs as much as hundreds of them
   if (*done || (seq && ++*polls % 1024)) {
     return TEMPI_SUCCESS;
   }
-  const hipError_t q = hipStreamQuery(library_stream());
+  const hipError_t q =
+      !seq && ev ? hipEventQuery(ev) : hipStreamQuery(library_stream());
   if (q == hipErrorNotReady) {
     return TEMPI_SUCCESS;
   }
@@ -843,11 +861,12 @@ int poll_signal_or_stream(unsigned long long seq, uint32_t *polls, bool *done) {
                : set_error(TEMPI_ERR_HIP, "a copy ended without its signal");
 }
 
-int wait_signal_or_stream(unsigned long long seq) {
+int wait_signal_or_stream(unsigned long long seq, hipEvent_t ev) {
   if (seq) {
     return wait_signal(signal_state(), seq);
   }
-  TEMPI_HIP_CHECK(hipStreamSynchronize(library_stream()));
+  TEMPI_HIP_CHECK(ev ? hipEventSynchronize(ev)
+                     : hipStreamSynchronize(library_stream()));
   return TEMPI_SUCCESS;
 }
 

@@ -355,6 +355,7 @@ class IsendOp : public AsyncOp {
   enum { PACKING, SENDING, DONE } state_ = PACKING;
   Staging stg_;
   unsigned long long seq_ = 0; // the pack's completion signal (0: none)
+  hipEvent_t ev_ = nullptr;    // an event behind the pack instead
   bool own_ = false;           // the pack's own workgroups send it
   uint32_t polls_ = 0;
   MPI_Request lib_req_ = MPI_REQUEST_NULL;
@@ -376,6 +377,9 @@ public:
       // never completed (an error path): the pack may still be running
       (void)hipStreamSynchronize(library_stream());
     }
+    if (ev_) {
+      (void)hipEventDestroy(ev_);
+    }
     stg_.release();
   }
   bool is_send() const override { return true; }
@@ -389,6 +393,9 @@ public:
       err = enqueue_pack(cn, count, ubuf_dev, stg_, s);
       seq_ = err ? 0 : signal_stream();
     }
+    if (!err && !seq_) {
+      ev_ = mark_library_stream();
+    }
     return err;
   }
   int wake() override {
@@ -396,7 +403,7 @@ public:
       return MPI_SUCCESS;
     }
     bool done = false;
-    if (poll_signal_or_stream(seq_, &polls_, &done)) {
+    if (poll_signal_or_stream(seq_, ev_, &polls_, &done)) {
       TEMPI_LOG(LOG_ERROR, "pack for MPI_Isend: %s", tempi_last_error());
       return MPI_ERR_INTERN;
     }
@@ -410,7 +417,7 @@ public:
     if (state_ != PACKING) {
       return MPI_SUCCESS;
     }
-    if (wait_signal_or_stream(seq_)) {
+    if (wait_signal_or_stream(seq_, ev_)) {
       TEMPI_LOG(LOG_ERROR, "pack for MPI_Isend: %s", tempi_last_error());
       return MPI_ERR_INTERN;
     }
@@ -445,6 +452,7 @@ class IrecvOp : public AsyncOp {
   enum { RECEIVING, UNPACKING, DONE } state_ = RECEIVING;
   Staging stg_;
   unsigned long long seq_ = 0; // the unpack's completion signal (0: none)
+  hipEvent_t ev_ = nullptr;    // an event behind the unpack instead
   bool own_ = false;           // the unpack's own workgroups send it
   uint32_t polls_ = 0;
   MPI_Request lib_req_ = MPI_REQUEST_NULL;
@@ -471,6 +479,9 @@ class IrecvOp : public AsyncOp {
       err = enqueue_unpack(cn_, n, ubuf_dev_, stg_, (int64_t)n * cn_.size, s);
       seq_ = err ? 0 : signal_stream();
     }
+    if (!err && !seq_) {
+      ev_ = mark_library_stream();
+    }
     return mpi_error_of(err);
   }
 
@@ -480,6 +491,9 @@ public:
   ~IrecvOp() override {
     if (state_ == UNPACKING) {
       (void)hipStreamSynchronize(library_stream());
+    }
+    if (ev_) {
+      (void)hipEventDestroy(ev_);
     }
     stg_.release();
   }
@@ -509,7 +523,7 @@ public:
         return error_;
       }
       bool done = false;
-      if (poll_signal_or_stream(seq_, &polls_, &done)) {
+      if (poll_signal_or_stream(seq_, ev_, &polls_, &done)) {
         TEMPI_LOG(LOG_ERROR, "unpack for MPI_Irecv: %s", tempi_last_error());
         return MPI_ERR_INTERN;
       }
@@ -544,7 +558,7 @@ public:
       }
     }
     if (state_ == UNPACKING && error_ == MPI_SUCCESS) {
-      if (wait_signal_or_stream(seq_)) {
+      if (wait_signal_or_stream(seq_, ev_)) {
         TEMPI_LOG(LOG_ERROR, "unpack for MPI_Irecv: %s", tempi_last_error());
         error_ = MPI_ERR_INTERN;
       } else {
