@@ -314,8 +314,8 @@ struct Walk {
 //   20 MB 11.8 -> 11.8    16 GiB 16.1 -> 11.8    100 GiB 31.6 -> 11.7
 // and 1 000 packs of one 64-KiB region 17.2 -> 11.7.  Returns the length of the
 // occupied part.
-int64_t lay_out(const std::vector<Req> &rs, const std::vector<BatchItem> &items,
-                std::vector<Walk> *walk) {
+uint64_t lay_out(const std::vector<Req> &rs, const std::vector<BatchItem> &items,
+                 std::vector<Walk> *walk) {
   struct Range {
     uintptr_t first, last;
     size_t r;
@@ -349,19 +349,19 @@ int64_t lay_out(const std::vector<Req> &rs, const std::vector<BatchItem> &items,
     }
     w.cost = (float)(((double)touched_bytes(g) + (double)g.L * g.rows) / it.ntiles);
   }
-  return (int64_t)(end - left_out);
+  return end - left_out;
 }
 
 void order_tiles(const std::vector<Req> &rs, const std::vector<BatchItem> &items,
                  uint64_t tiles, int groups, Tile *out, uint32_t *begin) {
   const size_t n = items.size();
   std::vector<Walk> walk(n);
-  const int64_t span = lay_out(rs, items, &walk);
+  const uint64_t span = lay_out(rs, items, &walk);
   int shift = kWindowShift;
-  while ((uint64_t)(span >> shift) > 2 * tiles + 1024) {
+  while ((span >> shift) > 2 * tiles + 1024) {
     ++shift;
   }
-  const int64_t windows = (span >> shift) + 1;
+  const int64_t windows = (int64_t)(span >> shift) + 1;
   std::vector<uint32_t> at((size_t)windows + 1, 0);
   const auto window = [&](int64_t pos) {
     return std::min(std::max<int64_t>(pos >> (shift + 12), 0), windows - 1);
@@ -1166,14 +1166,13 @@ TEMPI_EXPORT int tempi_batch_run_noalloc(const tempi_batch_request *reqs,
   return TEMPI_SUCCESS;
 }
 
+namespace {
+
 // What tempi_batch_run_noalloc would launch for requests whose addresses are
 // numbers: the same plan, read back from the tables' host image.
-TEMPI_EXPORT int tempi_batch_emulate(const tempi_batch_request *reqs, int64_t n,
-                                     int packed_on_host, int32_t *variants,
-                                     tempi_batch_emulation *out) {
-  if ((n > 0 && !reqs) || n < 0 || !out) {
-    return set_error(TEMPI_ERR_ARG, "bad argument");
-  }
+int emulate_batch(const tempi_batch_request *reqs, int64_t n,
+                  bool packed_on_host, int32_t *variants,
+                  tempi_batch_emulation *out) {
   *out = tempi_batch_emulation{};
   Resolved q;
   BatchPlan pl;
@@ -1182,7 +1181,7 @@ TEMPI_EXPORT int tempi_batch_emulate(const tempi_batch_request *reqs, int64_t n,
       [&](const tempi_batch_request &r, Req *rq) {
         rq->ds = static_cast<const char *>(r.strided);
         rq->dp = static_cast<char *>(r.packed);
-        rq->g.host = packed_on_host != 0;
+        rq->g.host = packed_on_host;
         return true;
       },
       &q, &pl);
@@ -1245,4 +1244,19 @@ TEMPI_EXPORT int tempi_batch_emulate(const tempi_batch_request *reqs, int64_t n,
   out->exact = inside && std::all_of(runs.begin(), runs.end(),
                                      [](uint8_t c) { return c == 1; });
   return TEMPI_SUCCESS;
+}
+
+} // namespace
+
+TEMPI_EXPORT int tempi_batch_emulate(const tempi_batch_request *reqs, int64_t n,
+                                     int packed_on_host, int32_t *variants,
+                                     tempi_batch_emulation *out) {
+  if ((n > 0 && !reqs) || n < 0 || !out) {
+    return set_error(TEMPI_ERR_ARG, "bad argument");
+  }
+  try {
+    return emulate_batch(reqs, n, packed_on_host != 0, variants, out);
+  } catch (const std::bad_alloc &) {
+    return set_error(TEMPI_ERR_NOMEM, "no host memory for the batch plan");
+  }
 }
