@@ -47,10 +47,11 @@ constexpr uint32_t kXcds = 8;
 // 254 unpacks of 4-B rows 4 - 516 B apart took 799 us with two, 1 013 us with
 // four, 238 of 8-B rows 421 and 509 us.  A batch of few requests has the device
 // to itself, and its unpacks take four: the three faces of a 512^3 float grid,
-// unpack alone, 8.3 us with two, 7.7 with four.  Its packs, whose loads of a
-// line each then queue behind each other, take two (8.8 us; 9.4 with four), and
-// so do requests of less than 3/4 of a tile per CU, for twice the workgroups
-// (pack + unpack, 320^3, 100 tiles of four: 11.1 us; 11.6 with four).
+// unpack alone, 8.3 us with two, 7.7 with four (of a 448^3 grid the same).  Its
+// packs, whose loads of a line each then queue behind each other, take two
+// (8.8 us; 9.4 with four), and so do requests of less than 3/4 of a tile per
+// CU, for twice the workgroups (pack + unpack, 320^3, 100 tiles of four: 11.1
+// us; 11.6 with four).
 __host__ __device__ constexpr bool two_or_four(int P, int U) {
   return P == 1 && units_in_flight(U) > 2;
 }

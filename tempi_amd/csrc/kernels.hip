@@ -276,8 +276,24 @@ static int plain_variant(int v) {
 //
 // A nontemporal store that covers part of a 64-B sector goes to memory by
 // itself, where a cached one waits in the Infinity Cache for its neighbours:
-// short rows never take them, rows that cut sectors only when their lines
-// could not stay cached anyway.  Then the packed stream is read nontemporal
+// rows under 16 B never take them, rows that cut sectors only when their lines
+// could not stay cached anyway.  Pack then unpack, three buffer sets in turn,
+// by the lines of the strided side, cached -> this rule, us:
+//   lines of                     300 MiB      600 MiB
+//   16-B rows 700 B apart       197 -> 170   396 -> 331
+//   64-B rows 192 B apart, 4 B  237 -> 179   482 -> 367
+//     past a line
+//   144-B rows 200 B apart      313 -> 243   607 -> 610
+//   256-B rows 700 B apart      281 -> 216   531 -> 483
+//   512-B rows 1088 B apart     284 -> 188   549 -> 459
+//   4-KiB rows 8256 B apart     259 -> 255   524 -> 509
+// An unpack alone ends later for it, as its stores have reached memory by then,
+// where cached ones leave up to 256 MiB of dirty lines to whatever runs next.
+// 300 MiB of lines, one unpack after the caches were emptied / one followed by
+// a kernel that reads the grid: 64 B at 192 B 37 -> 56 / 106 -> 110, 256 B cut
+// 107 -> 143 / 254 -> 194, 4 KiB at 4160 B 94 -> 115 / 185 -> 175.
+//
+// Short rows that cut sectors below that read the packed stream nontemporal
 // instead, which leaves the cache to those lines.  And a line that two
 // instructions read nontemporal is fetched twice: rows must be covered by
 // one access of a group, or be long.  (600 000 rows of 100 B at 1138 B, 96 B
@@ -345,14 +361,17 @@ int heuristic_variant(const Geom &g, const char *strided, const char *packed,
 // launch cadence (2.2-2.6 us on MI355X), which leaves the selector nothing to
 // rank; waited for, the one with the fewest workgroups and the widest words
 // that cut no row is seen first.  MPI_Pack, us (workgroups):
-//   1024 rows of 256 B   variant 4 9.5 (32), 10 9.7 (64), 1 10.7 (256)
-//   8192 rows of 64 B    variant 6 10.0 (64), 4 10.4 (256), 9 11.8 (128)
-//   1024 rows of 1 KiB   variant 4 10.1 (64), 1 10.3 (256), 7 11.3 (64)
-//   4096 rows of 24 B    variant 8 10.4 (32), 10 11.3 (512), 1 12.6 (2048)
-//   300 rows of 12 B     variants 9, 12 9.0 (2, 1), 7 9.8 (2), 1 10.6 (75)
-// Rows under 64 B leave this regime earlier: the kernel's own time shows
-// (64 Ki rows of 12 B: variants 9 11.3, 12 11.9, 4 12.7, 1 21.9 us), so beyond
-// 128 KiB they stay with the selector.
+//   1024 rows of 256 B   variant 4 10.3 (32), 10 10.3 (64), 1 10.6 (256)
+//   8192 rows of 64 B    variant 6 10.6 (64), 4 11.0 (256), 9 11.0 (128)
+//   1024 rows of 1 KiB   variant 4 10.6 (64), 1 10.8 (256), 7 10.9 (64)
+//   4096 rows of 48 B    variant 6 10.0 (32), 7 10.1 (16), 10 10.5 (256)
+//   4096 rows of 24 B    variant 8 10.1 (16), 10 10.8 (256), 4 10.9 (128)
+//   300 rows of 12 B     variants 12 9.1 (1), 9 9.6 (2), 4 10.5 (10)
+// Rows under 64 B beyond 128 KiB stay with the selector, which has caught up by
+// 512 KiB.  Eight row lengths of 4 - 48 B, rule and selector: 128 KiB 10.6 and
+// 10.8 us (packs), 11.0 and 11.2 (unpacks); 192 - 256 KiB between 0.8 better
+// and 0.3 worse; 512 KiB the same for packs, 11.6 and 11.5 for unpacks (12-B
+// rows 12.3 and 11.6).
 int latency_variant(const Geom &g) {
   const int64_t L = g.L, bytes = g.L * g.rows;
   if (bytes > (L < 64 ? 128ll << 10 : 1ll << 20)) {
