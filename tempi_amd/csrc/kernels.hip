@@ -300,33 +300,54 @@ static int plain_variant(int v) {
 // in 16-B words and a 4-B tail, one buffer set: cached 68 us per pass, loads
 // on both sides 86; 24-B rows as three 8-B words of a lane: 93, as one word
 // of three lanes: 64.)
+//
+// Where several short rows share a line, what counts is how many of them one
+// instruction reads: the 12-B words' kernel, a row per lane and four rows in
+// flight, or for 16-B rows the 8-B words' reads a line before it is evicted;
+// several lanes to a row (15, 17) or one row per lane with its words in turn
+// (18) read it again.  The same is seen below 64 MiB in rows under 8 B, which
+// are one or two accesses there, from 4 Mi rows on (1 - 2 Mi: from 14 % ahead of
+// variant 9 to 12 % behind it).  Pack then unpack, three sets in turn, us:
+//   24 MiB in 2-B rows 3 B apart     variant 9 91, 11 103, 12 59
+//   40 MiB in 4-B rows 8 B apart     18 88, 16 62, 9 80
+//   120 MiB in 8-B rows 12 B apart   17 195, 16 147, 8 149
+//   120 MiB in 16-B rows 20 B apart  15 160, 18 129, 7 123
+//   24 MiB in 8-B rows 64 B apart    17 143, 18 124, 16 128
+// Rows of 12 and 24 B nearly a line apart, each on a line of its own and part
+// of its neighbour's, are read cached once the lines outnumber the cache
+// (24 B 100 B apart, 500 MiB of lines: loads nontemporal 415, cached 385).
 int streamed_variant(int variant, const Geom &g, const char *strided, int dir,
                      int64_t touched) {
   const int plain = plain_variant(variant);
+  const int64_t L = g.L, apart = g.nrd ? std::abs(g.str[0]) : 0;
+  // several rows to a line, over many lines
+  const bool dense = g.nrd && apart < 32 && g.cnt[0] * apart >= 4096;
+  const bool word = L == 1 || L == 2 || L == 4 || L == 8;
   if (touched < kStreamBytes) {
-    return plain;
+    return dense && touched && L < 8 && apart < 24 && g.rows >= 4 << 20 ? 12
+                                                                        : plain;
   }
   // the packed address does not matter: the strided one stands in for it
   const bool sectors = geom_aligned(g, strided, strided + g.start, 64);
   const bool stores =
-      dir == TEMPI_DIR_UNPACK && g.L >= 16 &&
+      dir == TEMPI_DIR_UNPACK && L >= 16 &&
       (touched > kInfinityCache || (sectors && touched >= kInfinityCache / 2));
-  if (g.L > 512 || (g.L % 16 == 0 && g.L > 128)) {
+  if (L > 512 || (L % 16 == 0 && L > 128)) {
     return stores ? 2 : 3;
   }
-  if (g.L % 16 == 0) {
-    return g.L > 64 ? (stores ? 0 : 13) : (stores ? 14 : 15);
-  }
-  if (g.L == 12) {
+  if (dense && (word || L == 12 || (L < 8 && apart < 16))) {
     return 16;
   }
-  if (g.L % 8 == 0 && g.L <= 32) {
-    return 17;
-  }
-  if (g.L == 1 || g.L == 2 || g.L == 4) {
+  if (dense && L == 16) {
     return 18;
   }
-  return plain;
+  if (L % 16 == 0) {
+    return L > 64 ? (stores ? 0 : 13) : (stores ? 14 : 15);
+  }
+  if (apart >= 96 && apart < 128 && touched > kInfinityCache) {
+    return plain;
+  }
+  return L == 12 ? 16 : L == 24 ? 17 : word ? 18 : plain;
 }
 
 int heuristic_variant(const Geom &g, const char *strided, const char *packed,
