@@ -342,7 +342,7 @@ typedef struct tempi_batch_emulation {
   int64_t tiles;         /* workgroup passes                                */
   int64_t grid;          /* workgroups of the launch                        */
   int64_t xcd_tiles[8];  /* tiles that run on each XCD                      */
-  double xcd_bytes[8];   /* bytes of lines they move                        */
+  double xcd_cost[8];    /* what they are taken to cost, in bytes           */
   int32_t exact;         /* 1: every tile of every request runs once        */
   int32_t fits_static_tables;
 } tempi_batch_emulation;

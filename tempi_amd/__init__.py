@@ -152,7 +152,7 @@ class BatchEmulation(ctypes.Structure):
         ("tiles", ctypes.c_int64),
         ("grid", ctypes.c_int64),
         ("xcd_tiles", ctypes.c_int64 * 8),
-        ("xcd_bytes", ctypes.c_double * 8),
+        ("xcd_cost", ctypes.c_double * 8),
         ("exact", ctypes.c_int32),
         ("fits_static_tables", ctypes.c_int32),
     ]
@@ -547,7 +547,7 @@ def batch_emulate(requests, packed_on_host: bool = False) -> dict:
     check(lib().tempi_batch_emulate(arr, n, int(packed_on_host), variants, ctypes.byref(out)),
           "batch_emulate")
     r = {name: getattr(out, name) for name, _ in out._fields_}
-    return dict(r, xcd_tiles=list(out.xcd_tiles), xcd_bytes=list(out.xcd_bytes),
+    return dict(r, xcd_tiles=list(out.xcd_tiles), xcd_cost=list(out.xcd_cost),
                 variants=list(variants[:n]))
 
 

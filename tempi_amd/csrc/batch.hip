@@ -274,7 +274,7 @@ struct BatchPlan {
 
 // The tile records of a batch in the order of the strided side's addresses,
 // to windows of 4 KiB, cut into `groups` consecutive ranges of about
-// equal traffic (begin[x] is the first tile of range x; a range may end inside
+// equal cost (begin[x] is the first tile of range x; a range may end inside
 // a window).  Requests of a batch share lines -- a halo's faces, edges and
 // corners, the low x face of a row and the high one of the row before -- and
 // partly written lines: with every request in turn, and an eighth of each on
@@ -304,8 +304,26 @@ void strided_range(const Req &q, uintptr_t *first, uintptr_t *last) {
 struct Walk {
   int64_t at;   // first tile's position, 12 fraction bits
   int64_t step; // from tile to tile, 12 fraction bits
-  float cost;   // bytes of lines a tile moves
+  float cost;   // tile_cost
 };
+
+// What a tile of a request takes of an XCD, in bytes of lines at about 0.67 per
+// ns: its lines and packed bytes, but no less than its workgroup's own time.
+// Batches of 40 requests of one row length, ns per tile of an XCD, measured
+// and as bytes: packs of rows of 16 B - 4 KiB 0.96 to 1.17 of each other (100 B
+// 1.33); 1-B rows 2 B apart 12.2 and 2.3 (2 KiB), 4-B rows 5 B apart 14.4 and
+// 6.9.  Unpacks whose rows cut sectors take half as much again (64-B rows 65 B
+// apart 38 and 25, 256 B 33 and 25), unless their packed bytes are read
+// nontemporal (1 000 B 46 and 48).
+float tile_cost(const Req &q, uint32_t ntiles) {
+  const Geom &g = q.g;
+  double bytes = ((double)touched_bytes(g) + (double)g.L * g.rows) / ntiles;
+  if (q.dir == TEMPI_DIR_UNPACK && g.L <= 512 &&
+      !geom_aligned(g, q.ds, q.ds + g.start, 64)) {
+    bytes *= 1.5;
+  }
+  return (float)std::max(bytes, 8192.0);
+}
 
 // The positions are the strided addresses with the memory between the
 // requests left out: two grids far apart would otherwise share the windows
@@ -323,15 +341,35 @@ uint64_t lay_out(const std::vector<Req> &rs, const std::vector<BatchItem> &items
   };
   const size_t n = items.size();
   std::vector<Range> ranges(n);
+  uintptr_t lo = UINTPTR_MAX, hi = 0;
   for (size_t r = 0; r < n; ++r) {
-    strided_range(rs[r], &ranges[r].first, &ranges[r].last);
-    ranges[r].r = r;
+    Range &q = ranges[r];
+    strided_range(rs[r], &q.first, &q.last);
+    q.r = r;
+    lo = std::min(lo, q.first);
+    hi = std::max(hi, q.last);
   }
-  std::sort(ranges.begin(), ranges.end(),
-            [](const Range &a, const Range &b) { return a.first < b.first; });
+  // sorted only where gaps may take half of the span or more, told by how many
+  // of its 64 parts a request reaches into
+  constexpr uintptr_t kParts = 64;
+  const uintptr_t part = (hi - lo) / kParts + 1;
+  int edges[kParts + 1] = {}, open = 0, occupied = 0;
+  for (const Range &q : ranges) {
+    ++edges[(q.first - lo) / part];
+    --edges[std::min((q.last - 1 - lo) / part + 1, kParts)];
+  }
+  for (uintptr_t k = 0; k < kParts; ++k) {
+    open += edges[k];
+    occupied += open > 0;
+  }
+  const bool gaps = occupied <= (int)kParts / 2;
+  if (gaps) {
+    std::sort(ranges.begin(), ranges.end(), [](const Range &a, const Range &b) {
+      return a.first < b.first;
+    });
+  }
   constexpr uintptr_t kWindow = (uintptr_t)1 << kWindowShift;
-  uintptr_t left_out = ranges[0].first / kWindow * kWindow;
-  uintptr_t end = ranges[0].first;
+  uintptr_t left_out = lo / kWindow * kWindow, end = gaps ? lo : hi;
   for (const Range &q : ranges) {
     if (q.first > end) {
       left_out += (q.first - end) / kWindow * kWindow;
@@ -348,7 +386,7 @@ uint64_t lay_out(const std::vector<Req> &rs, const std::vector<BatchItem> &items
     if (g.rows == 1) {
       w.step = (int64_t)((double)g.L * 4096 / it.ntiles);
     }
-    w.cost = (float)(((double)touched_bytes(g) + (double)g.L * g.rows) / it.ntiles);
+    w.cost = tile_cost(rs[q.r], it.ntiles);
   }
   return end - left_out;
 }
@@ -404,6 +442,8 @@ int plan_tables(const std::vector<Req> &rs, BatchPlan *pl) {
   std::vector<BatchItem> items;
   std::vector<uint32_t> item_tiles; // tiles of each item
   uint64_t tiles = 0;
+  items.reserve(rs.size());
+  item_tiles.reserve(rs.size());
   const bool small = rs.size() <= (size_t)kSmallItems;
   for (const Req &r : rs) {
     BatchItem it{};
@@ -544,6 +584,8 @@ int resolve_requests(const tempi_batch_request *reqs, int64_t n,
   if (on_device && (err = ensure_runtime())) {
     return err;
   }
+  out->rs.reserve((size_t)n);
+  out->where.reserve((size_t)n);
   for (int64_t i = 0; i < n; ++i) {
     const tempi_batch_request &r = reqs[i];
     Req q;
@@ -1216,11 +1258,9 @@ int emulate_batch(const tempi_batch_request *reqs, int64_t n,
       inside = false;
       return;
     }
-    const Geom &g = q.rs[r].g;
     runs[first[r] + l] += runs[first[r] + l] < 2;
     ++out->xcd_tiles[xcd];
-    out->xcd_bytes[xcd] +=
-        ((double)touched_bytes(g) + (double)g.L * g.rows) / items[r].ntiles;
+    out->xcd_cost[xcd] += tile_cost(q.rs[r], items[r].ntiles);
   };
   if (L.small) {
     for (uint32_t r = 0; r < L.ix.n; ++r) {

@@ -1,5 +1,5 @@
 """The tile plan of a batch, on the host: every tile of every request runs
-exactly once, and each of the eight XCDs gets an eighth of the traffic (to one
+exactly once, and each of the eight XCDs gets an eighth of the cost (to one
 tile) wherever the requests' buffers lie."""
 import random
 
@@ -55,23 +55,36 @@ def mixed():
     return reqs
 
 
-# bound of one tile's bytes: 1024 rows of a line each, both sides
-LARGEST_TILE = 1024 * (128 + 128) + 2 * 65536
+# bound of one tile's cost: 1024 rows of a line each, both sides, half as much again
+LARGEST_TILE = 1.5 * (1024 * (128 + 128) + 2 * 65536)
+
+
+def long_and_tiny_rows():
+    """Half of the tiles hold 4-KiB rows, the other half 1-B rows."""
+    long, tiny = rows2d(4096, 512, 4160), rows2d(1, 512 * 128, 2)
+    return [(sb, (1 << 40) + k * (4 << 20), (1 << 45) + (k << 22), 1, ta.DIR_PACK)
+            for k, sb in enumerate([long] * 20 + [tiny] * 20)]
 
 
 @pytest.mark.parametrize("make", [
     lambda: far_grids(16 * GIB), lambda: far_grids(100 * GIB), lambda: far_grids(-(1 << 39)),
-    one_window, same_face, sparse_and_dense, mixed,
-], ids=["16GiB", "100GiB", "below", "one_window", "same_face", "sparse", "mixed"])
+    one_window, same_face, sparse_and_dense, mixed, long_and_tiny_rows,
+], ids=["16GiB", "100GiB", "below", "one_window", "same_face", "sparse", "mixed", "long_tiny"])
 def test_every_xcd_gets_its_share(make):
     reqs = make()
     e = ta.batch_emulate(reqs)
     assert e["exact"] == 1 and e["requests"] == len(reqs)
     assert sum(e["xcd_tiles"]) == e["tiles"] >= 64
     assert e["grid"] == 8 * max(e["xcd_tiles"])
-    total = sum(e["xcd_bytes"])
-    assert max(e["xcd_bytes"]) <= total / 8 + LARGEST_TILE
-    assert min(e["xcd_bytes"]) >= total / 8 - LARGEST_TILE
+    total = sum(e["xcd_cost"])
+    assert max(e["xcd_cost"]) <= total / 8 + LARGEST_TILE
+    assert min(e["xcd_cost"]) >= total / 8 - LARGEST_TILE
+
+
+def test_a_workgroup_costs_something():
+    """Tiles of 1-B rows move 2 KiB and take a quarter of the time of 32-KiB ones."""
+    e = ta.batch_emulate(long_and_tiny_rows())
+    assert max(e["xcd_tiles"]) <= 5 * min(e["xcd_tiles"])
 
 
 @pytest.mark.parametrize("n", [1, 8, 9])
