@@ -204,7 +204,8 @@ int run(Exchange &e, MPI_Comm comm) {
     err = set_error(TEMPI_ERR_HIP, "staging copy failed");
   }
   if (!err) {
-    err = wait_library_stream();
+    err = e.method == TEMPI_METHOD_STAGED ? wait_host_copy(e.out.total)
+                                          : wait_library_stream();
   }
   if (err) {
     return MPI_ERR_INTERN;

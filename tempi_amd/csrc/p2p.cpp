@@ -391,7 +391,8 @@ public:
                                stg_.kernel_side(), stg_.kernel_host(), TEMPI_DIR_PACK, &seq_, &own_);
     } else if (!err) {
       err = enqueue_pack(cn, count, ubuf_dev, stg_, s);
-      seq_ = err ? 0 : signal_stream();
+      // (behind a copy by a DMA engine the event below: wait_host_copy)
+      seq_ = err || stg_.bytes >= kEngineCopy ? 0 : signal_stream();
     }
     if (!err && !seq_) {
       ev_ = mark_library_stream();
@@ -833,7 +834,7 @@ TEMPI_EXPORT int MPI_Send(const void *buf, int count, MPI_Datatype datatype,
   } else if (!terr) {
     terr = enqueue_pack(cn, count, dev, st, s);
     if (!terr) {
-      terr = wait_library_stream();
+      terr = wait_host_copy(st.bytes);
     }
   }
   if (terr) {

@@ -105,3 +105,36 @@ def test_the_copy_signals_itself_where_that_is_the_shorter_wait(mpi, block, rows
         o.unpack(want, ref, 0, 1)
         assert (fetch(lib, dst, n) == ref).all(), it
     mpi.free(h)
+
+
+@pytest.mark.parametrize("rows,kernels", [(64, 2), (256, 1), (2048, 1)])
+def test_a_copy_by_the_dma_engine_has_no_signal_kernel_behind_it(mpi, rows, kernels):
+    """STAGED: the send waits for its copy to the host with the stream where
+    that copy is larger than 16 KiB; the receive's unpack signals."""
+    ta.lib().tempi_set_datatype_method(3)
+    spec = ("vector", rows, 256, 300, tc.BYTE)
+    h = mpi.type_from_spec(spec)
+    o = orc.OracleType(spec)
+    n = o.span(1)[1]
+    src, dst = ta.DeviceBuffer(n), ta.DeviceBuffer(n)
+    try:
+        for it in range(5):
+            host = orc.splitmix_bytes(n, 500 + it)
+            src.upload(host)
+            dst.fill(0xAB)
+            ref = np.full(n, 0xAB, np.uint8)
+            o.unpack(o.pack(host, 0, 1), ref, 0, 1)
+            err, rr = mpi.irecv(dst.addr(), 1, h, 0, 91)
+            assert err == 0
+            k0 = ta.signals()[1]
+            if it % 2:
+                err, sr = mpi.isend(src.addr(), 1, h, 0, 91)
+                assert err == 0 and mpi.wait(sr, h)[0] == 0
+            else:
+                assert mpi.send(src.addr(), 1, h, 0, 91) == 0
+            assert mpi.wait(rr, h)[0] == 0
+            assert ta.signals()[1] - k0 == kernels, it
+            assert (dst.download() == ref).all(), it
+    finally:
+        ta.lib().tempi_set_datatype_method(-1)
+    mpi.free(h)
